@@ -1,0 +1,82 @@
+"""Prefill kernels at the edges of their tiles and splits, against the oracle.
+
+One-layer models: the 1B model's layer, whose GEMMs leave tiles in parts at
+these lengths, and one whose row counts are odd multiples of 64 (the last
+256-row tile is mostly past the edge).
+"""
+import dataclasses
+import os
+
+import numpy as np
+import pytest
+
+from conftest import model_root
+
+pytestmark = pytest.mark.gpu
+ABS_TOL, REL_TOL = 2e-3, 1e-3  # the logit tolerance of every parity test
+
+
+@pytest.fixture(scope="module")
+def mods():
+    import oracle.oracle as O
+    import tinyminigo_amd as T
+    from tinyminigo_amd import workloads as W
+
+    O.set_attn_threads(max(1, min(16, os.cpu_count() or 1)))
+    yield T, O, W
+    O.set_attn_threads(1)
+
+
+_open = {}
+
+
+def _models(mods, which):
+    if which not in _open:
+        T, O, W = mods
+        if which == "1b":
+            wl = dataclasses.replace(W.ONE_B, name="minicpm5-1b-synthetic-l1", num_hidden_layers=1)
+        elif which == "4b":
+            wl = dataclasses.replace(W.FOUR_B, name="minicpm5-4b-synthetic-l1", num_hidden_layers=1)
+        else:
+            wl = dataclasses.replace(W.ONE_B, name="llama-h1088-i2112-l1", num_hidden_layers=1, hidden_size=1088,
+                                     num_attention_heads=8, num_key_value_heads=4, intermediate_size=2112,
+                                     vocab_size=777, weight_seed=29)
+        p = W.ensure_model(wl, model_root())
+        _open[which] = T.Model.load(p), O.OracleModel.load(p), wl
+    return _open[which]
+
+
+def _close(a, b, what):
+    d = np.abs(np.asarray(a, np.float64) - np.asarray(b, np.float64))
+    assert np.all(d <= ABS_TOL + REL_TOL * np.abs(b)), f"{what}: max abs {d.max():.3e}"
+
+
+def _check(mods, which, pieces):
+    T, _, _ = mods
+    g, o, wl = _models(mods, which)
+    total = sum(pieces)
+    ids = [int(t) for t in T.synth_tokens(83, total, wl.vocab_size)]
+    gc, oc = T.KvCache(g, total), o.new_cache()
+    at, first = 0, None
+    for n in pieces:
+        print(f"{which} prefill {n} at {at}", flush=True)
+        a = g.forward_seq(ids[at:at + n], gc)
+        first = a if first is None else first
+        _close(a, o.forward_seq(ids[at:at + n], oc), f"{which} prefill {n} at {at}")
+        at += n
+    _close(gc.keys_flat(0), oc.keys_flat(0), "keys")
+    _close(gc.values_flat(0), oc.values_flat(0), "values")
+    # the order of every sum is fixed: a rerun is bitwise identical
+    gc2 = T.KvCache(g, total)
+    assert np.array_equal(first, g.forward_seq(ids[:pieces[0]], gc2))
+    gc.close()
+    gc2.close()
+
+
+# the tiled GEMM over spans of K steps: one token past a tile, a whole number
+# of tiles, past the short-prompt kernel's range, and lengths where spans cross
+# tiles and where tiles stay whole
+@pytest.mark.parametrize("which,n", [("1b", 257), ("1b", 577), ("1b", 640), ("1b", 1025), ("1b", 1408),
+                                     ("h1088", 577), ("h1088", 1100)])
+def test_tiled_gemm_spans(mods, which, n):
+    _check(mods, which, [n])

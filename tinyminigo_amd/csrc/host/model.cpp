@@ -667,7 +667,7 @@ static int ensure_prefill(tmg_model *m, int T) {
         return rc;
     if (!m->pf_part) {
         const size_t nc = skinny_counters(std::max(std::max(m->qkv_rows, m->H), 2 * m->I));
-        if ((rc = dev_alloc(m, &m->pf_part, kSkinnyPartFloats)) || (rc = dev_alloc(m, &m->pf_cnt, nc))) return rc;
+        if ((rc = dev_alloc(m, &m->pf_part, kGemmPartFloats)) || (rc = dev_alloc(m, &m->pf_cnt, nc))) return rc;
         hipError_t e = hipMemset(m->pf_cnt, 0, nc * sizeof(unsigned));
         if (e != hipSuccess) return set_error(TMG_E_DEVICE, std::string("hipMemset: ") + hipGetErrorString(e));
     }

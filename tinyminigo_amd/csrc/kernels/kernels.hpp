@@ -244,19 +244,23 @@ struct GemmArgs {
     unsigned *cnt;
 };
 
-// Prompts of at least kTiledMinTokens tokens (and K a multiple of 64) use the
-// LDS-tiled 128x128 kernel; shorter ones the 64x64 split-K kernel (K a
-// multiple of 64) or the 16x64 streaming kernel.
+// Prompts of at least kTiledMinTokens tokens may take the 256 x 256 GEMM tile,
+// and their attention the MFMA kernel; up to kShortMaxTokens tokens the
+// split-K kernel of short prompts (launch_gemm chooses by estimated time).
 constexpr int kTiledMinTokens = 256;
+constexpr int kShortMaxTokens = 1024;
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s);
 // Whether launch_gemm takes a kernel whose output goes through
 // stage_epilogue for these shapes (the only ones that honour nrm_w / nss_in).
 bool gemm_stages_output(int M, int N, int K);
 constexpr int kMaxNormGroups = 40;  // hidden sizes up to 2560 for the norm hand-off
-// Workspace the short-prompt kernel needs: floats of partials and counters
-// for any GEMM with at most `max_m` rows and fewer than kTiledMinTokens tokens.
+// Split-K workspace of launch_gemm: two partial 256 x 128 tiles for each of at
+// most kSpanSlots spans of the tiled kernel, or the short-prompt kernel's at
+// most 768 partial 64 x 64 tiles (its counters: one per 16 tokens of a tile).
+constexpr int kSpanSlots = 256;  // one workgroup per CU
 constexpr size_t kSkinnyPartFloats = (size_t)768 * 64 * 64;
-inline size_t skinny_counters(int max_m) { return (size_t)((max_m + 63) / 64) * ((kTiledMinTokens + 63) / 64) * 4; }
+constexpr size_t kGemmPartFloats = (size_t)kSpanSlots * 2 * 256 * 128;
+inline size_t skinny_counters(int max_m) { return (size_t)((max_m + 63) / 64) * (kShortMaxTokens / 64) * 4; }
 
 // Copy row `row` of x[T,H] to dst[H] (last prefill row -> decode residual).
 hipError_t launch_copy_row(const float *x, int row, int H, float *dst, hipStream_t s);

@@ -9,6 +9,9 @@
 // BF16 and accumulation is f32.  Epilogues fuse RoPE + KV append, the
 // residual add and SwiGLU; the next GEMM's split operands are written
 // directly.
+#include <algorithm>
+#include <cmath>
+
 #include "coh.cuh"
 #include "common.cuh"
 #include "kernels.hpp"
@@ -514,108 +517,240 @@ __global__ __launch_bounds__(kBlock) void gemm_f32w_kernel(const GemmArgs a) {
     gemm_store<EPI>(a, mb, n, v);
 }
 
-// Tiled MFMA GEMM for prompts of at least kTiledMinTokens tokens: workgroup
-// tile 128 weight rows x 128 tokens, K in steps of 64; each of the four
-// wavefronts owns a 64 x 64 quarter (4 x 4 MFMA fragments).
-constexpr int kTM = 128, kTN = 128, kTK = 64;
+constexpr int kGWaves = 8;  // wavefronts of the tiled kernels, two per SIMD
 
-// The W / Bhi / Blo tiles go global -> LDS directly (global_load_lds_dwordx4,
-// no register staging) through a 3-stage ring, so step s + 2 is in flight
-// while step s is multiplied and each step needs one barrier.  LDS rows are unpadded 128 B with the 16-byte chunks
-// XOR-swizzled by (row & 7) against bank conflicts: a DMA wave-instruction
-// fills 1 KB = 8 rows contiguously, so each lane fetches the global chunk that
-// belongs at its LDS slot.
-constexpr int kGStages = 3;
-constexpr int kGTile = kTM * kTK * 2;  // bytes of one 128 x 64 bf16 tile
+// Tiled MFMA GEMM over spans of K steps: workgroup tile 256 weight rows x 128
+// tokens, K in steps of 32.  The tiles' K steps, tile after tile, form one
+// line of tiles * nk units that is cut into gridDim.x equal spans, one per
+// workgroup, so the chip is evenly loaded whatever the tile count.  A span
+// that covers a whole tile ends in the epilogue; where a tile's steps belong
+// to several spans, each stores its partial tile and gemm_span_reduce_kernel,
+// launched behind, adds the partials in span order and runs the epilogue.
+//
+// Wave w owns rows 64 (w & 3) .. +63 and tokens 64 (w >> 2) .. +63 (4 x 4
+// MFMA fragments).  The W / Bhi / Blo tiles go global -> LDS by DMA through a
+// four-stage ring of 32 KB stages.  LDS rows are 64 B with their 16-byte
+// chunks XOR-swizzled as in gemm_big_kernel.
+constexpr int kTM = 256, kTN = 128, kTK = 32;
+constexpr int kTStages = 4;
+constexpr int kTWTile = kTM * kTK * 2, kTBTile = kTN * kTK * 2;  // bytes of one W / one B tile
+constexpr int kTStage = kTWTile + 2 * kTBTile;
 
-// NW = 8 wavefronts (two per SIMD, so one's MFMAs overlap the other's LDS
-// reads): wave w owns rows 64 (w & 1) .. +63 and tokens 32 (w >> 1) .. +31
-// (4 x 2 MFMA fragments) and issues two of each tile's 16 DMA instructions.
-constexpr int kGWaves = 8;
+// The cut of the line: span c is [start(c), start(c + 1)), the first `rem`
+// spans one unit longer than the others.
+struct SpanCut {
+    int n_tiles, nk, base, rem;
+    __device__ __forceinline__ int start(int c) const { return c * base + min(c, rem); }
+    __device__ __forceinline__ int span_of(int u) const {
+        const int big = rem * (base + 1);
+        return u < big ? u / (base + 1) : rem + (u - big) / base;
+    }
+    // span c's partial of the tile whose units begin at t0: a span holds at
+    // most two partial tiles, slot 1 the tile it ends in after starting in an
+    // earlier one
+    __device__ __forceinline__ size_t slot(int c, int t0) const { return (size_t)2 * c + (start(c) < t0 ? 1 : 0); }
+};
 
 template <int EPI>
-__global__ __launch_bounds__(kGWaves * 64) void gemm_dma_kernel(const GemmArgs a) {
-    constexpr int DPW = 16 / kGWaves;  // DMA instructions per wave per tile
-    constexpr int NJ = kTN / 16 / (kGWaves / 2);  // token fragments per wave
-    static_assert(3 * DPW <= 15, "vmcnt immediate");
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[kGStages * 3 * kGTile];
+__global__ __launch_bounds__(kGWaves * 64) void gemm_span_kernel(const GemmArgs a, const SpanCut cut) {
+    constexpr int WPW = kTWTile / 1024 / kGWaves, BPW = kTBTile / 1024 / kGWaves;  // DMA instructions per wave
+    constexpr int DPS = WPW + 2 * BPW;                                             // per step
+    constexpr int FI = 4, FJ = 4;
+    static_assert(BPW == 1 && kTStages == 4 && 3 * DPS <= 15, "DMA map and vmcnt immediates");
+    static_assert(kGWaves * FJ * 16 * kStagePitch * 4 <= kTStages * kTStage, "the output staging fits the ring");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[kTStages * kTStage];
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int m0 = blockIdx.x * kTM, n0 = blockIdx.y * kTN;
-    const int K = a.K;
-    const int nsteps = K / kTK;
-    // DMA: wave w's instruction i fills rows (DPW w + i) * 8 .. +7 of a tile;
-    // lane l writes row (DPW w + i) * 8 + (l >> 3), physical chunk l & 7, which
-    // holds logical chunk (l & 7) ^ (row & 7)
-    uint32_t off[3][DPW];
-#pragma unroll
-    for (int i = 0; i < DPW; i++) {
-        const int row = (wave * DPW + i) * 8 + (lane >> 3);
-        const int lc = (lane & 7) ^ (row & 7);
-        off[0][i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + lc * 8;
-        off[1][i] = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + lc * 8;
-        off[2][i] = off[1][i];
-    }
-    auto issue = [&](int stage, int k0) {
-#pragma unroll
-        for (int x = 0; x < 3; x++) {
-            const uint16_t *base = x == 0 ? a.W : (x == 1 ? a.Bhi : a.Blo);
-#pragma unroll
-            for (int i = 0; i < DPW; i++)
-                __builtin_amdgcn_global_load_lds(base + off[x][i] + k0,
-                                                 smem + (stage * 3 + x) * kGTile + (wave * DPW + i) * 1024, 16, 0, 0);
-        }
-    };
-    issue(0, 0);
-    if (nsteps > 1) issue(1, kTK);
-    f32x4 acc[4][NJ];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < NJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int wm = wave & 3, wn = wave >> 2;
     const int r = lane & 15, q4 = lane >> 4;
-    for (int st = 0; st < nsteps; st++) {
-        // this step's 3 DPW DMAs are complete once at most the next step's are
-        // outstanding (vector memory counts complete in issue order)
-        if (st + 1 < nsteps)
-            __builtin_amdgcn_s_waitcnt(0xF70 | (3 * DPW));  // vmcnt(3 DPW)
-        else
-            __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
-        __builtin_amdgcn_s_barrier();  // every wave's DMAs for this step landed; step - 1's reads are done
-        if (st + 2 < nsteps) issue((st + 2) % kGStages, (st + 2) * kTK);
-        const unsigned char *sa = smem + ((st % kGStages) * 3 + 0) * kGTile;
-        const unsigned char *sh = sa + kGTile, *sl = sa + 2 * kGTile;
+    const int K = a.K, nk = cut.nk;
+    // workgroups go to the XCDs round robin: each XCD takes one contiguous
+    // eighth of the line (tiles with the token index fastest), so a weight
+    // row is read into one XCD's L2
+    const int G = gridDim.x, xq = G >> 3, xr = G & 7, xcd = blockIdx.x & 7;
+    const int g = xcd * xq + min(xcd, xr) + ((int)blockIdx.x >> 3);
+    const int u1 = cut.start(g + 1);
+    int u = cut.start(g);
+
+    uint32_t ao[FI], bo[FJ];
 #pragma unroll
-        for (int kk = 0; kk < kTK; kk += 32) {
-            const int lc = kk / 8 + q4;
-            bf16x8 fa[4], fh[NJ], fl[NJ];
+    for (int i = 0; i < FI; i++) {
+        const int ra = wm * 64 + i * 16 + r;
+        ao[i] = ra * 64 + ((q4 ^ ((ra >> 1) & 3)) * 16);
+    }
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int ra = wm * 64 + i * 16 + r;
-                fa[i] = *reinterpret_cast<const bf16x8 *>(sa + ra * 128 + ((lc ^ (ra & 7)) * 16));
-            }
+    for (int j = 0; j < FJ; j++) {
+        const int rb = wn * 64 + j * 16 + r;
+        bo[j] = kTWTile + rb * 64 + ((q4 ^ ((rb >> 1) & 3)) * 16);
+    }
+    auto rd = [&](int stage, uint32_t o) { return *reinterpret_cast<const bf16x8 *>(smem + stage * kTStage + o); };
+
+    while (u < u1) {
+        const int tile = u / nk, k0 = u - tile * nk;
+        const int ns = min(nk - k0, u1 - u);
+        u += ns;
+        const int mt = tile / cut.n_tiles, nt = tile - mt * cut.n_tiles;
+        const int m0 = mt * kTM, n0 = nt * kTN;
+        // a DMA wave-instruction fills 16 rows: rows 16 (2 wave + i) .. of W,
+        // 16 wave .. of Bhi and Blo
+        uint32_t woff[WPW], boff;
 #pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                const int rb = wn * NJ * 16 + j * 16 + r;
-                fh[j] = *reinterpret_cast<const bf16x8 *>(sh + rb * 128 + ((lc ^ (rb & 7)) * 16));
-                fl[j] = *reinterpret_cast<const bf16x8 *>(sl + rb * 128 + ((lc ^ (rb & 7)) * 16));
-            }
+        for (int i = 0; i < WPW; i++) {
+            const int row = (wave * WPW + i) * 16 + (lane >> 2);
+            woff[i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
+        }
+        {
+            const int row = wave * 16 + (lane >> 2);
+            boff = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
+        }
+        auto issue = [&](int st) {
+            unsigned char *dst = smem + (st % kTStages) * kTStage;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < WPW; i++)
+                __builtin_amdgcn_global_load_lds(a.W + woff[i] + st * kTK, dst + (wave * WPW + i) * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(a.Bhi + boff + st * kTK, dst + kTWTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(a.Blo + boff + st * kTK, dst + kTWTile + kTBTile + wave * 1024, 16, 0, 0);
+        };
+        // at most `n` later steps' DMAs may be outstanding (only DMAs are, and
+        // they complete in issue order)
+        auto wait_steps = [&](int n) {
+            if (n >= 3)
+                __builtin_amdgcn_s_waitcnt(0xF70 | (3 * DPS));
+            else if (n == 2)
+                __builtin_amdgcn_s_waitcnt(0xF70 | (2 * DPS));
+            else if (n == 1)
+                __builtin_amdgcn_s_waitcnt(0xF70 | DPS);
+            else
+                __builtin_amdgcn_s_waitcnt(0xF70);
+        };
+        // the previous tile's output stores are complete, so that the waits
+        // below count only DMAs, and its LDS staging has been read
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
 #pragma unroll
-                for (int j = 0; j < NJ; j++)
+        for (int st = 0; st < kTStages; st++)
+            if (st < ns) issue(st);
+        wait_steps(min(ns - 1, 3));
+        __builtin_amdgcn_s_barrier();
+        f32x4 acc[FI][FJ];
+#pragma unroll
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // a wavefront whose 64 rows or tokens all lie past the edge only
+        // moves data for the others
+        const bool live = n0 + wn * 64 < a.N && m0 + wm * 64 < a.M;
+        bf16x8 fa[FI], fh[FJ], fl[FJ];
+        if (live) {
+#pragma unroll
+            for (int i = 0; i < FI; i++) fa[i] = rd(0, ao[i]);
+#pragma unroll
+            for (int j = 0; j < FJ; j++) fh[j] = rd(0, bo[j]);
+        }
+        // as in gemm_big_kernel: the hi pass reads step st's Blo fragments,
+        // the lo pass step st + 1's W and Bhi fragments
+        auto hi_pass = [&](int stage) {
+#pragma unroll
+            for (int i = 0; i < FI; i++) {
+#pragma unroll
+                for (int j = 0; j < FJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fh[j], acc[i][j], 0, 0, 0);
+                if (i == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+                    for (int j = 0; j < FJ; j++) fl[j] = rd(stage, bo[j] + kTBTile);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        for (int st = 0; st + 1 < ns; st++) {
+            const int nx = (st + 1) % kTStages;
+            if (live) hi_pass(st % kTStages);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of stage st are done
+            wait_steps(min(ns - 2 - st, 2));     // step st + 1's DMAs have landed
+            __builtin_amdgcn_s_barrier();
+            if (st + kTStages < ns) issue(st + kTStages);
+            if (live) {
 #pragma unroll
-                for (int j = 0; j < NJ; j++)
+                for (int j = 0; j < FJ; j++) fh[j] = rd(nx, bo[j]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < FI; i++) {
+#pragma unroll
+                    for (int j = 0; j < FJ; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fl[j], acc[i][j], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fa[i] = rd(nx, ao[i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        if (live) {
+            hi_pass((ns - 1) % kTStages);
+#pragma unroll
+            for (int i = 0; i < FI; i++)
+#pragma unroll
+                for (int j = 0; j < FJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fl[j], acc[i][j], 0, 0, 0);
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // the ring is free for the output staging
+        asm volatile("" ::: "memory");
+        if (!live) continue;
+        if (ns < nk) {
+            f32x4 *part = reinterpret_cast<f32x4 *>(a.part) +
+                          (cut.slot(g, tile * nk) * kGWaves + wave) * (FI * FJ * 64) + lane;
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+#pragma unroll
+                for (int i = 0; i < FI; i++) part[(j * FI + i) * 64] = acc[i][j];
+        } else {
+            stage_epilogue<EPI, FI, FJ, 1>(a, reinterpret_cast<float *>(smem) + wave * FJ * 16 * kStagePitch,
+                                           m0 + wm * 64, n0 + wn * 64, acc);
+        }
     }
-    // the ring is free once every wave is past its last fragment reads
-    __builtin_amdgcn_s_barrier();
-    stage_epilogue<EPI, 4, NJ, 1>(a, reinterpret_cast<float *>(smem) + wave * NJ * 16 * kStagePitch, m0 + wm * 64,
-                               n0 + wn * NJ * 16, acc);
+}
+
+// The tiles that gemm_span_kernel left in parts: one wavefront per 64 rows x
+// 16 tokens (32 per tile) adds the spans' partials in span order and runs the
+// epilogue.
+template <int EPI>
+__global__ __launch_bounds__(kBlock) void gemm_span_reduce_kernel(const GemmArgs a, const SpanCut cut) {
+    __shared__ __attribute__((aligned(16))) float stage[4 * 16 * kStagePitch];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int item = blockIdx.x * 4 + wave;
+    const int tile = item >> 5, wreg = (item >> 2) & 7, j = item & 3;  // wave region of the tile, its token fragment
+    const int t0 = tile * cut.nk;
+    const int c0 = cut.span_of(t0), c1 = cut.span_of(t0 + cut.nk - 1);
+    const int mt = tile / cut.n_tiles, nt = tile - mt * cut.n_tiles;
+    const int mw = mt * kTM + (wreg & 3) * 64, nw = nt * kTN + (wreg >> 2) * 64 + j * 16;
+    if (c0 == c1 || mw >= a.M || nw >= a.N) return;
+    EpiPre<EPI, 4> pre;
+    epi_prefetch<EPI, 4>(a, mw, nw, pre);
+    const f32x4 *const part = reinterpret_cast<const f32x4 *>(a.part) + lane;
+    f32x4 acc[4][1];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int NC = 6;  // spans in flight
+#pragma unroll 1
+    for (int c = c0; c <= c1; c += NC) {
+        f32x4 v[NC][4];
+#pragma unroll
+        for (int x = 0; x < NC; x++)
+            if (c + x <= c1) {
+                const f32x4 *p = part + (cut.slot(c + x, t0) * kGWaves + wreg) * 1024 + j * 256;
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[x][i] = p[i * 64];
+            }
+#pragma unroll
+        for (int x = 0; x < NC; x++)
+            if (c + x <= c1)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][0][e] += v[x][i][e];
+    }
+    stage_epilogue<EPI, 4, 1, 4, true>(a, stage + wave * 16 * kStagePitch, mw, nw, acc, &pre);
 }
 
 // Large-tile MFMA GEMM for long prompts: workgroup tile 256 weight rows x
@@ -1075,6 +1210,15 @@ __global__ __launch_bounds__(2 * kBlock, 1) void gemm_skinny_wide_kernel(const G
                                        out, &pre);
 }
 
+// K splits of gemm_skinny_wide_kernel
+int skinny_wide_splits(const GemmArgs &a) {
+    const int m2 = (a.M + 127) / 128, n_tiles = (a.N + 63) / 64, nk = a.K / 64;
+    int ns = 1;
+    if (a.part && a.cnt)
+        while (ns * 2 <= kSkMaxSplit && nk / (ns * 2) >= 2 && m2 * n_tiles * ns * 2 <= 256) ns *= 2;
+    return ns;
+}
+
 hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
     // split K while the grid stays within one workgroup per CU, or while
     // splits keep at least 20 K steps within three workgroups per CU; at most
@@ -1122,9 +1266,7 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
     // split while the grid stays within one workgroup (eight waves, a 96 KB
     // ring) per CU
     const int m2 = (a.M + 127) / 128;
-    int ns2 = 1;
-    if (a.part && a.cnt)
-        while (ns2 * 2 <= kSkMaxSplit && nk / (ns2 * 2) >= 2 && m2 * n_tiles * ns2 * 2 <= 256) ns2 *= 2;
+    const int ns2 = skinny_wide_splits(a);
     if (ns2 > 1 && (size_t)m_tiles * n_tiles * ns2 * 4096 > kSkinnyPartFloats) return hipErrorInvalidValue;
     const dim3 grid2((m2 * ns2 + 7) / 8 * n_tiles * 8);
     switch (epi) {
@@ -1132,6 +1274,69 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
         case GEPI_RESID: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_RESID>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
         case GEPI_SWIGLU: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_SWIGLU>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
         case GEPI_QKV: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_QKV>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <int EPI>
+void launch_span_epi(const GemmArgs &a, const SpanCut &cut, int tiles, int G, hipStream_t s) {
+    hipLaunchKernelGGL(gemm_span_kernel<EPI>, dim3(G), dim3(kGWaves * 64), 0, s, a, cut);
+    if (G != tiles) hipLaunchKernelGGL(gemm_span_reduce_kernel<EPI>, dim3(tiles * 8), dim3(kBlock), 0, s, a, cut);
+}
+
+// Estimated microseconds of a GEMM on the three kernels that take more than
+// 64 tokens, from kernel traces of the 1B and 4B shapes at 75-8192 tokens.
+// Each is a fixed cost (launch, ring fill, epilogue) plus the K steps of the
+// longest workgroup: a 32-wide step of the 256 x 128 tile takes 0.9-1.1 us, of
+// the 256 x 256 tile 1.8, a 64-wide step of the 128 x 64 tile 0.6-0.75; a
+// K split of the short-prompt kernel costs about 5 us for its exchange, one
+// of the span kernel about 10 us plus 0.06 us per span (128 KB of partials
+// written and read back).  Choosing by them instead of by token count alone
+// (256 x 256 from 240 tiles, 128 x 128 from 256 tokens) takes the 1B prefill
+// from 6.6 to 3.95 ms at 301 tokens, 7.0 to 4.5 at 500, 8.3 to 7.3 at 1000,
+// 11.9 to 10.9 at 1500 and 20.7 to 19.0 at 3001, and leaves 100, 2000, 4096
+// and 8192 as they were.
+double big_us(const GemmArgs &a) {
+    const int wg = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
+    return 8.0 + 1.8 * ((wg + 255) / 256) * (a.K / kBK);
+}
+
+double skinny_wide_us(const GemmArgs &a) {
+    const int ns = skinny_wide_splits(a), wg = ((a.M + 127) / 128) * ((a.N + 63) / 64) * ns;
+    return 6.0 + (ns > 1 ? 5.0 : 0.0) + 0.7 * ((wg + 255) / 256) * (a.K / 64 / ns);
+}
+
+// Spans of a GEMM on gemm_span_kernel: the tile count (whole tiles), or as
+// many equal spans as the estimate makes best, at least 4 steps each.
+struct SpanPlan {
+    int spans;
+    double us;
+};
+
+SpanPlan plan_span(const GemmArgs &a) {
+    const int tiles = ((a.M + kTM - 1) / kTM) * ((a.N + kTN - 1) / kTN), nk = a.K / kTK;
+    const int64_t units = (int64_t)tiles * nk;
+    SpanPlan p{tiles, 6.0 + (double)((tiles + kSpanSlots - 1) / kSpanSlots) * nk};
+    if (a.part)
+        for (int g = 32; g <= kSpanSlots && units >= 4 * g; g += 16) {
+            const double us = 16.0 + (double)((units + g - 1) / g) + 0.06 * g;
+            if (us < p.us) p = SpanPlan{g, us};
+        }
+    return p;
+}
+
+hipError_t launch_span(int epi, const GemmArgs &a, hipStream_t s) {
+    const int m_tiles = (a.M + kTM - 1) / kTM, n_tiles = (a.N + kTN - 1) / kTN, nk = a.K / kTK;
+    const int tiles = m_tiles * n_tiles;
+    if ((int64_t)tiles * nk > 0x3fffffff) return hipErrorInvalidValue;
+    const int units = tiles * nk, G = plan_span(a).spans;
+    const SpanCut cut{n_tiles, nk, units / G, units % G};
+    switch (epi) {
+        case GEPI_STORE: launch_span_epi<GEPI_STORE>(a, cut, tiles, G, s); break;
+        case GEPI_RESID: launch_span_epi<GEPI_RESID>(a, cut, tiles, G, s); break;
+        case GEPI_SWIGLU: launch_span_epi<GEPI_SWIGLU>(a, cut, tiles, G, s); break;
+        case GEPI_QKV: launch_span_epi<GEPI_QKV>(a, cut, tiles, G, s); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1157,10 +1362,14 @@ hipError_t launch_rmsnorm_split(const float *x, const float *w, float eps, int T
     return hipGetLastError();
 }
 
+// Where K is an odd number of 32-wide steps: the 256 x 256 tile once its grid
+// is about a workgroup per CU.
+static bool big_fills(int M, int N) { return ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) >= 240; }
+
 bool gemm_stages_output(int M, int N, int K) {
-    if (K % 32 != 0 || M <= 0 || N <= 0) return false;
-    if (N >= kTiledMinTokens && ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) >= 240) return true;
-    return K % 64 == 0;  // the 128 x 128 tiled or the split-K kernel
+    if (M <= 0 || N <= 0) return false;
+    // every kernel of whole 64-wide K steps does, and the 256 x 256 tile
+    return K % 64 == 0 || (K % 32 == 0 && N >= kTiledMinTokens && big_fills(M, N));
 }
 
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
@@ -1181,8 +1390,10 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     if ((a.nrm_w || a.nss_in) && !gemm_stages_output(a.M, a.N, a.K)) return hipErrorInvalidValue;
     if (a.nrm_w && (epi != GEPI_RESID || a.M % 64 != 0 || !a.nss || !a.nx_hi || !a.nx_lo)) return hipErrorInvalidValue;
     if (a.nss_in && (a.ngroups <= 0 || a.ngroups > kMaxNormGroups || a.ngroups % 4)) return hipErrorInvalidValue;
-    // the 256 x 256 tile once its grid is about a workgroup per CU
-    if (a.N >= kTiledMinTokens && a.K % kBK == 0 && ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN) >= 240) {
+    const bool tiled = a.K % 64 == 0 && a.N > 64;
+    const double span_us = tiled ? plan_span(a).us : HUGE_VAL;
+    const double short_us = tiled && a.N <= kShortMaxTokens ? skinny_wide_us(a) : HUGE_VAL;
+    if (a.N >= kTiledMinTokens && (tiled ? big_us(a) < std::min(span_us, short_us) : big_fills(a.M, a.N))) {
         const dim3 grid((a.M + kBM - 1) / kBM, (a.N + kBN - 1) / kBN);
         switch (epi) {
             case GEPI_STORE: hipLaunchKernelGGL(gemm_big_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
@@ -1193,17 +1404,7 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
         }
         return hipGetLastError();
     }
-    if (a.N >= kTiledMinTokens && a.K % kTK == 0) {
-        const dim3 grid((a.M + kTM - 1) / kTM, (a.N + kTN - 1) / kTN);
-        switch (epi) {
-            case GEPI_STORE: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_RESID: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_QKV: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    }
+    if (tiled && span_us < short_us) return launch_span(epi, a, s);
     if (a.K % 64 == 0) return launch_skinny(epi, a, s);
     const dim3 grid((a.M + 15) / 16, (a.N + 63) / 64);
     switch (epi) {
