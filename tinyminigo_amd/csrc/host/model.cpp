@@ -773,6 +773,10 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
         if (m->nq / m->nkv >= 4) aa.block = attn_chunk(m->hd, m->nq / m->nkv, kAttnThreads, kAttnBlockShort);
         aa.out_hi = m->pf_ahi;
         aa.out_lo = m->pf_alo;
+        // the GEMMs' split workspace is free between them
+        static_assert(kGemmPartFloats >= (size_t)kAttnRuns * 128 * (128 + 2), "attention runs fit the workspace");
+        aa.part = m->pf_part;
+        aa.part_ml = m->pf_part + (size_t)kAttnRuns * 128 * 128;
         if (attn_prefill_supported(aa)) {
             if ((rc = ensure_kv_split(m, start + T))) return rc;
             KVSplitArgs ka{kc, vc, start + T, m->nkv, m->hd, m->pf_kh, m->pf_kl, m->pf_vth, m->pf_vtl, m->kv_cap};

@@ -23,6 +23,13 @@
 // kv_split_kernel (V transposed per head), so the attention workgroups stage
 // ready-made MFMA operands: each block's 64 KB are plain 16-byte copies, and
 // the next block's copies are in flight while the current one is multiplied.
+//
+// Where the query blocks alone leave CUs idle, a query block's key blocks are
+// dealt to several workgroups in contiguous runs (AttnArgs::key_run); each
+// writes its unnormalized output with its running maximum and sum, and
+// attn_prefill_combine_kernel merges them in key order.
+#include <algorithm>
+
 #include "common.cuh"
 #include "kernels.hpp"
 
@@ -152,6 +159,23 @@ __device__ __forceinline__ void dma16(const uint16_t *src, unsigned char *dst) {
     __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
 }
 
+// Key blocks of query block qb (the context of its last row), and the
+// workgroups they are dealt to, at most `run` blocks each.
+__host__ __device__ inline int key_blocks(int start, int T, int QB, int qb) {
+    const int last = start + (T < (qb + 1) * QB ? T : (qb + 1) * QB) - 1;
+    return last / kPKB + 1;
+}
+__host__ __device__ inline int key_splits(int nkb, int run) { return (nkb + run - 1) / run; }
+
+// Four consecutive output dims as split-bf16.
+__device__ __forceinline__ void store_split4(const f32x4 &v, uint16_t *hi, uint16_t *lo) {
+    uint16_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) split_bf16(v[i], h + i, l + i);
+    *reinterpret_cast<u32x2 *>(hi) = u32x2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+    *reinterpret_cast<u32x2 *>(lo) = u32x2{(uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16)};
+}
+
 template <int GROUP>
 __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnArgs a) {
     constexpr int QB = kPCols / GROUP;  // query positions per workgroup
@@ -164,7 +188,22 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
     // XCD streams only its heads' K/V through its L2
     const int nqb = (a.T + QB - 1) / QB;
     const int g = (int)blockIdx.x % a.nkv;
-    const int qb = nqb - 1 - (int)blockIdx.x / a.nkv;
+    int qb = nqb - 1 - (int)blockIdx.x / a.nkv, sp = 0, nsp = 1;
+    int kb0 = 0, kb1 = 0;
+    if (a.key_run) {
+        // the same order with each query block's runs next to each other
+        sp = (int)blockIdx.x / a.nkv;
+        for (qb = nqb - 1; qb >= 0; qb--) {
+            nsp = key_splits(key_blocks(a.start, a.T, QB, qb), a.key_run);
+            if (sp < nsp) break;
+            sp -= nsp;
+        }
+    }
+    {
+        const int n = key_blocks(a.start, a.T, QB, qb);
+        kb0 = sp * n / nsp;
+        kb1 = (sp + 1) * n / nsp;
+    }
     const int kvd = a.nkv * kPHD, qd = a.nq * kPHD;
 
     // this lane's query column in each of its 16-column tiles
@@ -177,8 +216,10 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
         qpos[qt] = a.start + ti[qt];
         qhead[qt] = g * GROUP + hh;
     }
-    const int last_pos = a.start + min(a.T, (qb + 1) * QB) - 1;  // the workgroup's last query position
-    const int nkb = last_pos / kPKB + 1;
+    // a wavefront whose query columns all lie past the last row only moves data
+    bool live = false;
+#pragma unroll
+    for (int qt = 0; qt < kPQT; qt++) live = live || __builtin_amdgcn_ballot_w64(ti[qt] < a.T) != 0;
 
     // Q is pre-scaled by scale / ln 2, so the scores come out in log2 units
     const float sl2 = a.scale * 1.4426950408889634f;
@@ -300,7 +341,7 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, s[kt][qt][i]);
-            mx = max_xor16_32(mx);  // finite: key 0 precedes every query
+            mx = max_xor16_32(mx);  // -inf while a run of keys lies past the query
             const bool raise = mx > m[qt] + 8.0f;
             if (__builtin_amdgcn_ballot_w64(raise)) {
                 const float corr = raise ? __builtin_amdgcn_exp2f(m[qt] - mx) : 1.0f;
@@ -309,11 +350,12 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
 #pragma unroll
                 for (int dt = 0; dt < 8; dt++) o[qt][dt] *= corr;
             }
+            const float ref = m[qt] == -INFINITY ? 0.0f : m[qt];
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = __builtin_amdgcn_exp2f(s[kt][qt][i] - m[qt]);
+                    const float p = __builtin_amdgcn_exp2f(s[kt][qt][i] - ref);
                     s[kt][qt][i] = p;
                     l[qt] += p;
                 }
@@ -363,51 +405,116 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
     // issued in iteration kb - 1, waited for (vmcnt 0, only DMAs are
     // outstanding) before the barrier that also retires every wave's reads
     // of the stages K(kb + 2) and V(kb + 1) then overwrite.
-    issue_k(0);
-    issue_v(0);
-    if (nkb > 1) issue_k(1);
+    issue_k(kb0);
+    issue_v(kb0);
+    if (kb0 + 1 < kb1) issue_k(kb0 + 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     f32x4 sc[2][4][kPQT];
-    scores(0, sc[0]);
+    if (live) scores(kb0, sc[0]);
     const bool scores_first = wave < 4;
     auto iteration = [&](int kb, f32x4 (&cur)[4][kPQT], f32x4 (&nxt)[4][kPQT]) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (kb + 2 < nkb) issue_k(kb + 2);
-        if (kb + 1 < nkb) issue_v(kb + 1);
+        if (kb + 2 < kb1) issue_k(kb + 2);
+        if (kb + 1 < kb1) issue_v(kb + 1);
+        if (!live) return;
         if (scores_first) {
-            if (kb + 1 < nkb) scores(kb + 1, nxt);
+            if (kb + 1 < kb1) scores(kb + 1, nxt);
             softmax(kb, cur);
         } else {
             softmax(kb, cur);
-            if (kb + 1 < nkb) scores(kb + 1, nxt);
+            if (kb + 1 < kb1) scores(kb + 1, nxt);
         }
         accumulate(kb, cur);
     };
-    int kb = 0;
-    for (; kb + 1 < nkb; kb += 2) {
+    int kb = kb0;
+    for (; kb + 1 < kb1; kb += 2) {
         iteration(kb, sc[0], sc[1]);
         iteration(kb + 1, sc[1], sc[0]);
     }
-    if (kb < nkb) iteration(kb, sc[0], sc[1]);
-    // normalize and write the split-bf16 output: O^T rows dims 16 dt + 4 q4 + i
+    if (kb < kb1) iteration(kb, sc[0], sc[1]);
+    if (!live) return;
+    // normalize and write the split-bf16 output (O^T rows dims 16 dt + 4 q4 +
+    // i), or with several runs the unnormalized output, maximum and sum
 #pragma unroll
     for (int qt = 0; qt < kPQT; qt++) {
         const float L = add_xor32(add_xor16(l[qt]));  // the column's four lane groups
+        if (nsp > 1) {
+            const size_t tile = ((size_t)blockIdx.x * kPWaves + wave) * kPQT + qt;
+            f32x4 *part = reinterpret_cast<f32x4 *>(a.part) + tile * 512 + lane;
+#pragma unroll
+            for (int dt = 0; dt < 8; dt++) part[dt * 64] = o[qt][dt];
+            if (q4 == 0) *reinterpret_cast<float2 *>(a.part_ml + (tile * 16 + r) * 2) = make_float2(m[qt], L);
+            continue;
+        }
         if (ti[qt] >= a.T) continue;
         const float inv = 1.0f / L;
-        const size_t ob = (size_t)ti[qt] * qd + qhead[qt] * kPHD;
+        const size_t ob = (size_t)ti[qt] * qd + qhead[qt] * kPHD + 4 * q4;
 #pragma unroll
         for (int dt = 0; dt < 8; dt++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int d = dt * 16 + 4 * q4 + i;
-                split_bf16(o[qt][dt][i] * inv, a.out_hi + ob + d, a.out_lo + ob + d);
-            }
+            const f32x4 v = o[qt][dt] * inv;
+            store_split4(v, a.out_hi + ob + dt * 16, a.out_lo + ob + dt * 16);
         }
+    }
+}
+
+// Merges the runs of one 16-column tile of a query block: one workgroup per
+// (query block, wavefront of attn_prefill_kernel, KV head), each of its four
+// wavefronts two of the tile's eight 16-dim slices, the runs in key order.
+template <int GROUP>
+__global__ __launch_bounds__(kBlock) void attn_prefill_combine_kernel(const AttnArgs a) {
+    static_assert(kPQT == 1, "one query tile per wavefront");
+    constexpr int QB = kPCols / GROUP;
+    const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
+    const int dt0 = (threadIdx.x >> 6) * 2;
+    const int g = (int)blockIdx.x % a.nkv, w = (int)blockIdx.x / a.nkv % kPWaves;
+    const int nqb = (a.T + QB - 1) / QB;
+    const int qb = nqb - 1 - (int)blockIdx.x / (a.nkv * kPWaves);
+    const int c = w * 16 + r, hh = c / QB, ti = qb * QB + c - hh * QB;
+    int first = 0;
+    for (int b = nqb - 1; b > qb; b--) first += key_splits(key_blocks(a.start, a.T, QB, b), a.key_run);
+    const int nsp = key_splits(key_blocks(a.start, a.T, QB, qb), a.key_run);
+    if (nsp == 1 || __builtin_amdgcn_ballot_w64(ti < a.T) == 0) return;
+    float M = -INFINITY, L = 0.0f;
+    f32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr int NC = 8;  // runs in flight
+#pragma unroll 1
+    for (int s = 0; s < nsp; s += NC) {
+        float2 ml[NC];
+        f32x4 v[NC][2];
+#pragma unroll
+        for (int x = 0; x < NC; x++)
+            if (s + x < nsp) {
+                const size_t tile = ((size_t)(first + s + x) * a.nkv + g) * kPWaves + w;
+                ml[x] = *reinterpret_cast<const float2 *>(a.part_ml + (tile * 16 + r) * 2);
+                const f32x4 *part = reinterpret_cast<const f32x4 *>(a.part) + tile * 512 + dt0 * 64 + lane;
+                v[x][0] = part[0];
+                v[x][1] = part[64];
+            }
+#pragma unroll
+        for (int x = 0; x < NC; x++)
+            if (s + x < nsp) {
+                // the first run holds key 0, so M is finite from then on
+                const float nm = fmaxf(M, ml[x].x);
+                const float f0 = __builtin_amdgcn_exp2f(M - nm), f1 = __builtin_amdgcn_exp2f(ml[x].x - nm);
+                M = nm;
+                L = L * f0 + ml[x].y * f1;
+#pragma unroll
+                for (int d = 0; d < 2; d++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) o[d][i] = o[d][i] * f0 + v[x][d][i] * f1;
+            }
+    }
+    if (ti >= a.T) return;
+    const float inv = 1.0f / L;
+    const size_t ob = (size_t)ti * (a.nq * kPHD) + (g * GROUP + hh) * kPHD + dt0 * 16 + 4 * q4;
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+        const f32x4 v = o[d] * inv;
+        store_split4(v, a.out_hi + ob + d * 16, a.out_lo + ob + d * 16);
     }
 }
 
@@ -420,25 +527,84 @@ hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+namespace {
+
+// Workgroups and estimated microseconds of the MFMA attention with at most
+// `run` key blocks per workgroup (0: whole query blocks).  A 64-key block
+// takes a workgroup 2.9 us (one workgroup per CU; longest first, so the last
+// round is about half full where there are more), launch and first loads
+// 6 us; merging runs is a second launch, 6 us, and 64 KB of partials per
+// workgroup written and read back.
+struct AttnPlan {
+    int run, workgroups;
+    double us;
+};
+
+AttnPlan cost_attn(const AttnArgs &a, int QB, int run) {
+    const int nqb = (a.T + QB - 1) / QB;
+    int64_t wgs = 0, blocks = 0;
+    int longest = 0;
+    for (int qb = 0; qb < nqb; qb++) {
+        const int n = key_blocks(a.start, a.T, QB, qb), ns = run ? key_splits(n, run) : 1;
+        wgs += ns;
+        blocks += n;
+        longest = std::max(longest, (n + ns - 1) / ns);
+    }
+    wgs *= a.nkv;
+    blocks *= a.nkv;
+    const double us = 6.0 + 2.9 * (wgs <= 256 ? (double)longest : std::max((double)longest, blocks / 256.0 + 0.5 * longest)) +
+                      (run ? 6.0 + 0.03 * wgs : 0.0);
+    return AttnPlan{run, (int)std::min<int64_t>(wgs, 1 << 30), us};
+}
+
+AttnPlan plan_attn(const AttnArgs &a) {
+    const int group = a.nq / a.nkv, QB = kPCols / group;
+    AttnPlan best = cost_attn(a, QB, 0);
+    if (!a.part || !a.part_ml || best.workgroups > 2 * kAttnRuns) return best;
+    const int most = key_blocks(a.start, a.T, QB, (a.T + QB - 1) / QB - 1);
+    for (int run = 1; run < most; run += 1 + run / 8) {
+        const AttnPlan p = cost_attn(a, QB, run);
+        if (p.workgroups <= kAttnRuns && p.us < best.us) best = p;
+    }
+    return best;
+}
+
+template <int GROUP>
+void launch_attn_prefill_group(AttnArgs a, hipStream_t s) {
+    const AttnPlan p = plan_attn(a);
+    a.key_run = p.run;
+    hipLaunchKernelGGL(attn_prefill_kernel<GROUP>, dim3(p.workgroups), dim3(kPWaves * 64), 0, s, a);
+    const int nqb = (a.T + kPCols / GROUP - 1) / (kPCols / GROUP);
+    if (p.run)
+        hipLaunchKernelGGL(attn_prefill_combine_kernel<GROUP>, dim3(nqb * kPWaves * a.nkv), dim3(kBlock), 0, s, a);
+}
+
+}  // namespace
+
 bool attn_prefill_supported(const AttnArgs &a) {
     const int group = a.nkv > 0 ? a.nq / a.nkv : 0;
-    // short prompts keep the per-row kernel: a few query blocks cannot fill the chip
-    return a.hd == kPHD && a.out_hi && a.out_lo && a.nq == group * a.nkv && a.T >= kTiledMinTokens &&
-           (group == 1 || group == 2 || group == 4 || group == 8);
+    if (a.hd != kPHD || !a.out_hi || !a.out_lo || a.nq != group * a.nkv ||
+        !(group == 1 || group == 2 || group == 4 || group == 8))
+        return false;
+    if (a.T >= kTiledMinTokens) return true;
+    // Below, the per-row kernel (T nkv workgroups, each over the whole
+    // context) where it is estimated faster: 1.66 us per 64 positions of one
+    // round, 200 such chunks per us once the chip is full.  The MFMA path also
+    // splits the cached rows into bf16 pairs (5.5 us + 2.4 ns per position).
+    const double chunks = (a.start + a.T + 63) / 64;
+    const double rows_us = 3.0 + std::max(1.66 * chunks, (double)a.T * a.nkv * chunks / 200.0);
+    return plan_attn(a).us + 5.5 + 0.0024 * (a.start + a.T) < rows_us;
 }
 
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s) {
     if (!attn_prefill_supported(a) || a.T <= 0 || !a.kh || !a.kl || !a.vth || !a.vtl ||
         a.vt_pitch < (a.start + a.T + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)
         return hipErrorInvalidValue;
-    const int group = a.nq / a.nkv;
-    const int QB = kPCols / group;
-    const dim3 grid(((a.T + QB - 1) / QB) * a.nkv);
-    switch (group) {
-        case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(kPWaves * 64), 0, s, a); break;
-        case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(kPWaves * 64), 0, s, a); break;
-        case 4: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, dim3(kPWaves * 64), 0, s, a); break;
-        case 8: hipLaunchKernelGGL(attn_prefill_kernel<8>, grid, dim3(kPWaves * 64), 0, s, a); break;
+    switch (a.nq / a.nkv) {
+        case 1: launch_attn_prefill_group<1>(a, s); break;
+        case 2: launch_attn_prefill_group<2>(a, s); break;
+        case 4: launch_attn_prefill_group<4>(a, s); break;
+        case 8: launch_attn_prefill_group<8>(a, s); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

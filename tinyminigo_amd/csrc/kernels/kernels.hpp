@@ -130,6 +130,9 @@ struct AttnArgs {
     // [pos][nkv*hd] and values transposed [nkv][hd][vt_pitch]
     const uint16_t *kh, *kl, *vth, *vtl;
     int vt_pitch;
+    // set by launch_attn_prefill: most key blocks per workgroup (0: all); part
+    // and part_ml then hold the runs of up to kAttnRuns workgroups
+    int key_run;
 };
 
 // Split-bf16 copies of one layer's KV cache rows [0, n) for the MFMA prefill
@@ -145,7 +148,10 @@ hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s);
 
 hipError_t launch_attn(const AttnArgs &a, hipStream_t s);
 // Causal prefill attention on MFMA (head_dim 128, split-bf16 output): the
-// shapes it takes, and the launch.
+// shapes it takes where it is the faster kernel, and the launch.  With a.part
+// (kAttnRuns x 128 x 128 floats) and a.part_ml (kAttnRuns x 128 x 2) a query
+// block's keys may be dealt to several workgroups.
+constexpr int kAttnRuns = 448;
 bool attn_prefill_supported(const AttnArgs &a);
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s);
 // Merges the split-K partials of a decode attention launch (a.T rows) into
