@@ -82,11 +82,11 @@ def test_tiled_gemm_spans(mods, which, n):
     _check(mods, which, [n])
 
 
-# the MFMA attention with a query block's keys dealt to several workgroups:
-# one row and a partial block after a long context, context and piece lengths
-# at and past the 64-key block, runs of one block (whole runs past some of the
-# queries), and whole query blocks
-@pytest.mark.parametrize("which,pieces", [("1b", [959, 1, 64]), ("1b", [1000, 45, 130, 300]), ("1b", [64, 63, 200, 65]),
-                                          ("1b", [320]), ("4b", [700, 33, 2, 128])])
+# attention with a query block's keys dealt to several workgroups: the fp32
+# kernel of pieces under 256 tokens (one row and a partial column tile after a
+# long context, pieces and contexts at and past the 64-key block, runs that
+# lie past some of the queries), the split-bf16 kernel above
+@pytest.mark.parametrize("which,pieces", [("1b", [959, 1, 64]), ("1b", [1000, 45, 130, 300]), ("1b", [448, 16, 17, 200, 65]),
+                                          ("1b", [320]), ("1b", [255, 255]), ("4b", [700, 33, 2, 128])])
 def test_attention_key_runs(mods, which, pieces):
     _check(mods, which, pieces)

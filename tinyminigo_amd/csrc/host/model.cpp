@@ -774,7 +774,8 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
         aa.out_hi = m->pf_ahi;
         aa.out_lo = m->pf_alo;
         // the GEMMs' split workspace is free between them
-        static_assert(kGemmPartFloats >= (size_t)kAttnRuns * 128 * (128 + 2), "attention runs fit the workspace");
+        static_assert(kGemmPartFloats >= (size_t)kAttnRuns * 128 * (128 + 2) && kAttnRuns * 128 >= kAttnF32Runs * 32,
+                      "attention runs fit the workspace");
         aa.part = m->pf_part;
         aa.part_ml = m->pf_part + (size_t)kAttnRuns * 128 * 128;
         if (attn_prefill_supported(aa)) {
@@ -787,6 +788,8 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
             aa.vtl = m->pf_vtl;
             aa.vt_pitch = m->kv_cap;
             TMG_HIP(launch_attn_prefill(aa, s));
+        } else if (attn_f32_pays(aa)) {
+            TMG_HIP(launch_attn_f32(aa, s));
         } else {
             TMG_HIP(launch_attn(aa, s));
         }

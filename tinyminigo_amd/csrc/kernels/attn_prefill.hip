@@ -586,14 +586,7 @@ bool attn_prefill_supported(const AttnArgs &a) {
     if (a.hd != kPHD || !a.out_hi || !a.out_lo || a.nq != group * a.nkv ||
         !(group == 1 || group == 2 || group == 4 || group == 8))
         return false;
-    if (a.T >= kTiledMinTokens) return true;
-    // Below, the per-row kernel (T nkv workgroups, each over the whole
-    // context) where it is estimated faster: 1.66 us per 64 positions of one
-    // round, 200 such chunks per us once the chip is full.  The MFMA path also
-    // splits the cached rows into bf16 pairs (5.5 us + 2.4 ns per position).
-    const double chunks = (a.start + a.T + 63) / 64;
-    const double rows_us = 3.0 + std::max(1.66 * chunks, (double)a.T * a.nkv * chunks / 200.0);
-    return plan_attn(a).us + 5.5 + 0.0024 * (a.start + a.T) < rows_us;
+    return a.T >= kTiledMinTokens;
 }
 
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s) {

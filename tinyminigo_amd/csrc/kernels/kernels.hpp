@@ -148,12 +148,19 @@ hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s);
 
 hipError_t launch_attn(const AttnArgs &a, hipStream_t s);
 // Causal prefill attention on MFMA (head_dim 128, split-bf16 output): the
-// shapes it takes where it is the faster kernel, and the launch.  With a.part
+// shapes it takes (at least kTiledMinTokens rows), and the launch.  With a.part
 // (kAttnRuns x 128 x 128 floats) and a.part_ml (kAttnRuns x 128 x 2) a query
 // block's keys may be dealt to several workgroups.
 constexpr int kAttnRuns = 448;
 bool attn_prefill_supported(const AttnArgs &a);
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s);
+// The same on the fp32 MFMA over the f32 cache, for fewer rows: whether it is
+// estimated faster than the per-row kernel, and the launch.  With a.part
+// (kAttnF32Runs x 32 x 128 floats) and a.part_ml (kAttnF32Runs x 32 x 2) a
+// column tile's keys may be dealt to several workgroups.
+constexpr int kAttnF32Runs = 512;
+bool attn_f32_pays(const AttnArgs &a);
+hipError_t launch_attn_f32(const AttnArgs &a, hipStream_t s);
 // Merges the split-K partials of a decode attention launch (a.T rows) into
 // out_f32 [T][nq*hd]: where the merge is not fused into the o_proj GEMV
 // prologue (more than kFusedSplits splits; batched decode).
