@@ -133,6 +133,19 @@ def test_batch_tied_and_k_not_multiple_of_64(T, O, W, tiny_path):
             assert got[b] == O.generate(o, p, 16).tokens, f"{path} sequence {b}"
 
 
+def test_batch_prompts_prefilled_together(T, O, untied):
+    # prompts under 256 tokens share prefills of up to 2048 rows: the first
+    # eight here fill 2040 of them, the one of 300 runs alone, the rest go into
+    # a second group; ids as the oracle's for every sequence
+    g, o, wl = untied
+    lens = [255] * 8 + [300, 64, 1, 2]
+    prompts = [[int(t) for t in T.synth_tokens(200 + i, n, wl.vocab_size)] for i, n in enumerate(lens)]
+    print("batch packed", lens, flush=True)
+    got, _ = T.generate_batch(g, prompts, 6)
+    for b, p in enumerate(prompts):
+        assert got[b] == O.generate(o, p, 6).tokens, f"sequence {b}"
+
+
 def test_batch_stops_each_sequence_at_eos(T, O, W, tiny_path, tmp_path):
     # an EOS id that sequence 0 emits mid-way: that sequence stops after it
     # (src/model.rs:649-651), the others run on

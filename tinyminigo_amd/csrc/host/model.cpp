@@ -688,20 +688,16 @@ static int ensure_kv_split(tmg_model *m, int n) {
     return TMG_OK;
 }
 
-// Runs the batched prefill; leaves the last token's logits in m->logits and
-// the per-workgroup argmax keys in m->argmax_part.
-int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
-    const int T = (int)n;
+// The layers of a batched prefill over T token rows, from m->pf_tokens to the
+// residual rows m->pf_x: one sequence at positions start .. in the cache k / v,
+// or with `rows` several, row n at position rows->pos[n] of the sequence whose
+// caches are rows->k[n] / rows->v[n].
+static int prefill_layers(tmg_model *m, int T, int start, float *k, float *v, uint32_t max_pos,
+                          const PrefillRows *rows) {
     const int H = m->H, I = m->I, qd = m->qd, kvd = m->kvd;
     hipStream_t s = m->stream;
     int rc;
-    if ((rc = ensure_prefill(m, T))) return rc;
-    if ((rc = ensure_rope(m, (int)c->len + T + 1))) return rc;
-    if ((rc = pinned(m, (size_t)T * 4 + 64 + (size_t)m->V * 4))) return rc;
-    memcpy(m->pin, tokens, (size_t)T * 4);
-    TMG_HIP(hipMemcpyAsync(m->pf_tokens, m->pin, (size_t)T * 4, hipMemcpyHostToDevice, s));
     TMG_HIP(launch_embed_gather(m->pf_tokens, T, H, m->embed_bf16, m->embed_f32, m->pf_x, s));
-    const int start = (int)c->len;
     const float eps = m->cfg.rms_norm_eps;
     // RMSNorm hand-off: the o_proj and down GEMMs write the next GEMM's
     // operand (new residual times the norm weight, split-bf16) and per-64-row
@@ -728,8 +724,9 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
     };
     for (int l = 0; l < m->L; l++) {
         const tmg_model::Layer &ly = m->layers[l];
-        float *kc = c->k + (size_t)l * c->max_pos * kvd;
-        float *vc = c->v + (size_t)l * c->max_pos * kvd;
+        const size_t layer_off = (size_t)l * max_pos * kvd;
+        float *kc = rows ? nullptr : k + layer_off;
+        float *vc = rows ? nullptr : v + layer_off;
         const bool in_handed = hand_off && l > 0;
         if (!in_handed) TMG_HIP(launch_rmsnorm_split(m->pf_x, ly.in_norm, eps, T, H, m->pf_hi, m->pf_lo, s));
         GemmArgs g{};
@@ -749,6 +746,12 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
         g.q_out = m->pf_q;
         g.k_cache = kc;
         g.v_cache = vc;
+        if (rows) {
+            g.pos_seq = rows->pos;
+            g.k_seq = rows->k;
+            g.v_seq = rows->v;
+            g.kv_layer_off = layer_off;
+        }
         g.part = m->pf_part;
         g.cnt = m->pf_cnt;
         if (m->i8) g.wscale = ly.qkv_s;
@@ -778,7 +781,13 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
                       "attention runs fit the workspace");
         aa.part = m->pf_part;
         aa.part_ml = m->pf_part + (size_t)kAttnRuns * 128 * 128;
-        if (attn_prefill_supported(aa)) {
+        if (rows) {
+            aa.pos_seq = rows->pos;
+            aa.k_seq = rows->k;
+            aa.v_seq = rows->v;
+            aa.kv_layer_off = layer_off;
+            TMG_HIP(launch_attn(aa, s));
+        } else if (attn_prefill_supported(aa)) {
             if ((rc = ensure_kv_split(m, start + T))) return rc;
             KVSplitArgs ka{kc, vc, start + T, m->nkv, m->hd, m->pf_kh, m->pf_kl, m->pf_vth, m->pf_vtl, m->kv_cap};
             TMG_HIP(launch_kv_split(ka, s));
@@ -841,18 +850,56 @@ int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
         if (hand_off && l + 1 < m->L) norm_out(d, m->layers[l + 1].in_norm);
         TMG_HIP(launch_gemm(GEPI_RESID, d, s));
     }
-    // final norm of the last row (batch association) + lm_head + argmax
+    return TMG_OK;
+}
+
+// Final norm of residual row `row` (batch association), lm_head and its
+// argmax keys.
+static int prefill_head(tmg_model *m, int row) {
+    const int H = m->H;
     GemvArgs la{};
     la.W = m->lm_head;
     la.Wf = m->lm_head_f;
     la.out = m->V;
     la.in = H;
-    la.x = m->pf_x + (size_t)(T - 1) * H;
+    la.x = m->pf_x + (size_t)row * H;
     la.norm_w = m->final_norm;
     la.eps = m->cfg.rms_norm_eps;
     la.y = m->logits;
     la.argmax_part = m->argmax_part;
-    TMG_HIP(launch_gemv(PRO_NORM_BATCH, EPI_LOGITS, la, s));
+    TMG_HIP(launch_gemv(PRO_NORM_BATCH, EPI_LOGITS, la, m->stream));
+    return TMG_OK;
+}
+
+// The prompt's ids to m->pf_tokens through the pinned staging buffer.
+static int stage_tokens(tmg_model *m, const uint32_t *tokens, size_t T) {
+    int rc;
+    if ((rc = ensure_prefill(m, (int)T))) return rc;
+    if ((rc = pinned(m, T * 4 + 64 + (size_t)m->V * 4))) return rc;
+    memcpy(m->pin, tokens, T * 4);
+    TMG_HIP(hipMemcpyAsync(m->pf_tokens, m->pin, T * 4, hipMemcpyHostToDevice, m->stream));
+    return TMG_OK;
+}
+
+int run_prefill_rows(tmg_model *m, const uint32_t *tokens, size_t n, uint32_t max_pos, const PrefillRows &rows) {
+    int rc;
+    if ((rc = stage_tokens(m, tokens, n))) return rc;
+    return prefill_layers(m, (int)n, 0, nullptr, nullptr, max_pos, &rows);
+}
+
+int run_prefill_head(tmg_model *m, int row) { return prefill_head(m, row); }
+
+// Runs the batched prefill; leaves the last token's logits in m->logits and
+// the per-workgroup argmax keys in m->argmax_part.
+int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n) {
+    const int T = (int)n;
+    hipStream_t s = m->stream;
+    int rc;
+    if ((rc = ensure_prefill(m, T))) return rc;
+    if ((rc = ensure_rope(m, (int)c->len + T + 1))) return rc;
+    if ((rc = stage_tokens(m, tokens, n))) return rc;
+    if ((rc = prefill_layers(m, T, (int)c->len, c->k, c->v, c->max_pos, nullptr))) return rc;
+    if ((rc = prefill_head(m, T - 1))) return rc;
     c->len += (uint32_t)T;
     // the device position follows the host mirror after a prefill
     memcpy((char *)m->pin + ((size_t)T * 4 + 63) / 64 * 64, &c->len, 4);

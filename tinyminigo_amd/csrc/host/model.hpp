@@ -175,6 +175,16 @@ bool step_graphs_enabled();
 int launch_step(tmg_model *m, tmg_cache *c, int mode, uint64_t pos);
 int set_state(tmg_model *m, tmg_cache *c, int token, bool reset_step);
 int run_prefill(tmg_model *m, tmg_cache *c, const uint32_t *tokens, size_t n);
+// Several sequences' prompts in one prefill: n token rows, row i at position
+// pos[i] (from 0) of the sequence whose caches [L][max_pos][kvd] are k[i] /
+// v[i] (device arrays; max_pos the same for all).  run_prefill_head then
+// leaves a row's logits and argmax keys as run_prefill does for its last row.
+struct PrefillRows {
+    const int *pos;
+    float *const *k, *const *v;
+};
+int run_prefill_rows(tmg_model *m, const uint32_t *tokens, size_t n, uint32_t max_pos, const PrefillRows &rows);
+int run_prefill_head(tmg_model *m, int row);
 int ensure_rope(tmg_model *m, int npos);
 int pinned(tmg_model *m, size_t bytes);
 
