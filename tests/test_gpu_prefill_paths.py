@@ -33,6 +33,12 @@ _open = {}
 def _models(mods, which):
     if which not in _open:
         T, O, W = mods
+        if which.startswith("f32-"):
+            from f32models import variant
+            wl = _models(mods, which[4:])[2]
+            p = variant(W.ensure_model(wl, model_root()), model_root(), "f32")
+            _open[which] = T.Model.load(p), O.OracleModel.load(p), wl
+            return _open[which]
         if which == "1b":
             wl = dataclasses.replace(W.ONE_B, name="minicpm5-1b-synthetic-l1", num_hidden_layers=1)
         elif which == "4b":
@@ -89,4 +95,12 @@ def test_tiled_gemm_spans(mods, which, n):
 @pytest.mark.parametrize("which,pieces", [("1b", [959, 1, 64]), ("1b", [1000, 45, 130, 300]), ("1b", [448, 16, 17, 200, 65]),
                                           ("1b", [320]), ("1b", [255, 255]), ("4b", [700, 33, 2, 128])])
 def test_attention_key_runs(mods, which, pieces):
+    _check(mods, which, pieces)
+
+
+# f32 weight matrices: the whole range of token counts takes the span kernel,
+# from one row (one live wavefront column) to several tiles
+@pytest.mark.parametrize("which,pieces", [("f32-1b", [1, 16]), ("f32-1b", [129, 64]), ("f32-1b", [640]),
+                                          ("f32-h1088", [2, 255]), ("f32-h1088", [300])])
+def test_f32_weight_gemm(mods, which, pieces):
     _check(mods, which, pieces)

@@ -463,60 +463,6 @@ __global__ __launch_bounds__(kBlock) void gemm_kernel(const GemmArgs a) {
     gemm_store<EPI>(a, mb, n, v);
 }
 
-// The same product over f32 weights (WMat::F32; matmul_batch_w_into's F32
-// arm, src/tensor.rs:573-760) on the fp32 MFMA v_mfma_f32_16x16x4_f32, whose
-// output layout is the bf16 one's: lane l supplies A row (l & 15) and B
-// column (l & 15) at k = l >> 4 and receives D rows 4 (l >> 4) .. +3 of
-// column (l & 15).  The activation is hi + lo, exact in f32.  Each lane
-// loads 4 consecutive k of its weight row and of its token (16 and 2 x 8
-// bytes), which serve 4 MFMAs: MFMA j takes the j-th of them from every lane,
-// the same k set on both operands.  Workgroup tile 16 rows x 64 tokens, the
-// four wavefronts on interleaved 16-wide K blocks, summed through LDS.
-template <int EPI>
-__global__ __launch_bounds__(kBlock) void gemm_f32w_kernel(const GemmArgs a) {
-    constexpr int NB = 4;  // 16-token column blocks per workgroup
-    __shared__ f32x4 s_acc[4][NB][64];
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16 * NB;
-    const int K = a.K;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    const float *Ap = a.Wf + (size_t)min(m0 + r, a.M - 1) * K + kq;
-    const uint16_t *Bh[NB], *Bl[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-        const int n = min(n0 + nb * 16 + r, a.N - 1);
-        Bh[nb] = a.Bhi + (size_t)n * K + kq;
-        Bl[nb] = a.Blo + (size_t)n * K + kq;
-    }
-    f32x4 acc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k = wave * 16; k < K; k += 64) {
-        const f32x4 av = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(Ap + k));
-        u32x2 bh[NB], bl[NB];
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            bh[nb] = *reinterpret_cast<const u32x2 *>(Bh[nb] + k);
-            bl[nb] = *reinterpret_cast<const u32x2 *>(Bl[nb] + k);
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const float x[4] = {bf16_lo(bh[nb].x) + bf16_lo(bl[nb].x), bf16_hi(bh[nb].x) + bf16_hi(bl[nb].x),
-                                bf16_lo(bh[nb].y) + bf16_lo(bl[nb].y), bf16_hi(bh[nb].y) + bf16_hi(bl[nb].y)};
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], x[j], acc[nb], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) s_acc[wave][nb][lane] = acc[nb];
-    __syncthreads();
-    const int nb = wave;
-    const f32x4 v = (s_acc[0][nb][lane] + s_acc[1][nb][lane]) + (s_acc[2][nb][lane] + s_acc[3][nb][lane]);
-    const int n = n0 + nb * 16 + (lane & 15);
-    const int mb = m0 + (lane >> 4) * 4;  // rows mb .. mb+3
-    gemm_store<EPI>(a, mb, n, v);
-}
-
 constexpr int kGWaves = 8;  // wavefronts of the tiled kernels, two per SIMD
 
 // Tiled MFMA GEMM over spans of K steps: workgroup tile 256 weight rows x 128
@@ -692,6 +638,153 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_span_kernel(const GemmArgs 
 #pragma unroll
                 for (int j = 0; j < FJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fl[j], acc[i][j], 0, 0, 0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // the ring is free for the output staging
+        asm volatile("" ::: "memory");
+        if (!live) continue;
+        if (ns < nk) {
+            f32x4 *part = reinterpret_cast<f32x4 *>(a.part) +
+                          (cut.slot(g, tile * nk) * kGWaves + wave) * (FI * FJ * 64) + lane;
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+#pragma unroll
+                for (int i = 0; i < FI; i++) part[(j * FI + i) * 64] = acc[i][j];
+        } else {
+            stage_epilogue<EPI, FI, FJ, 1>(a, reinterpret_cast<float *>(smem) + wave * FJ * 16 * kStagePitch,
+                                           m0 + wm * 64, n0 + wn * 64, acc);
+        }
+    }
+}
+
+// Eight f32 weights of a row as three bf16 parts that sum to them exactly:
+// the upper 8 significand bits by truncation, twice, and the rest.
+__device__ __forceinline__ void split3(const f32x4 &x0, const f32x4 &x1, bf16x8 (&p)[3]) {
+    uint32_t b[3][8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float x = i < 4 ? x0[i & 3] : x1[i & 3];
+        b[0][i] = __float_as_uint(x) & 0xffff0000u;
+        // an infinity is its first part alone (inf - inf is NaN)
+        const float r = fabsf(x) < INFINITY ? x - __uint_as_float(b[0][i]) : 0.0f;
+        b[1][i] = __float_as_uint(r) & 0xffff0000u;
+        b[2][i] = __float_as_uint(r - __uint_as_float(b[1][i]));
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        u32x4 u;
+#pragma unroll
+        for (int i = 0; i < 4; i++) u[i] = (b[k][2 * i] >> 16) | (b[k][2 * i + 1] & 0xffff0000u);
+        p[k] = __builtin_bit_cast(bf16x8, u);
+    }
+}
+
+// gemm_span_kernel over f32 weights (WMat::F32; matmul_batch_w_into's F32
+// arm, src/tensor.rs:573-760): the W tile is staged as f32 (128-byte rows,
+// chunks XOR-swizzled by row & 7, three 48 KB stages) and each fragment is
+// split into three bf16 parts in registers, so that six bf16 MFMAs give the
+// exact products of f32 weights and hi + lo activations: at 16 times the fp32
+// MFMA's rate, still faster than its four per 16 k.  It replaced an unstaged
+// 16 x 64 kernel on the fp32 MFMA, bound by L2 reads of its operands: four 1B
+// layers of F16 weights 1.20 -> 0.65 ms at 2 tokens, 1.69 -> 0.72 at 64, 3.48
+// -> 1.17 at 200, 14.2 -> 2.9 at 1000.
+constexpr int kFWTile = kTM * kTK * 4, kFStage = kFWTile + 2 * kTBTile, kFStages = 3;
+
+template <int EPI>
+__global__ __launch_bounds__(kGWaves * 64) void gemm_f32w_span_kernel(const GemmArgs a, const SpanCut cut) {
+    constexpr int WPW = kFWTile / 1024 / kGWaves;  // DMA instructions per wave of the W tile, 8 rows each
+    constexpr int DPS = WPW + 2;
+    constexpr int FI = 4, FJ = 4;
+    static_assert(kTBTile / 1024 == kGWaves && kFStages == 3 && 2 * DPS <= 15, "DMA map and vmcnt immediates");
+    static_assert(kGWaves * FJ * 16 * kStagePitch * 4 <= kFStages * kFStage, "the output staging fits the ring");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[kFStages * kFStage];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int wm = wave & 3, wn = wave >> 2;
+    const int r = lane & 15, q4 = lane >> 4;
+    const int K = a.K, nk = cut.nk;
+    const int G = gridDim.x, xq = G >> 3, xr = G & 7, xcd = blockIdx.x & 7;
+    const int g = xcd * xq + min(xcd, xr) + ((int)blockIdx.x >> 3);
+    const int u1 = cut.start(g + 1);
+    int u = cut.start(g);
+    uint32_t ao[FI][2], bo[FJ];
+#pragma unroll
+    for (int i = 0; i < FI; i++) {
+        const int ra = wm * 64 + i * 16 + r;
+#pragma unroll
+        for (int c = 0; c < 2; c++) ao[i][c] = ra * 128 + (((2 * q4 + c) ^ (ra & 7)) * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < FJ; j++) {
+        const int rb = wn * 64 + j * 16 + r;
+        bo[j] = kFWTile + rb * 64 + ((q4 ^ ((rb >> 1) & 3)) * 16);
+    }
+    while (u < u1) {
+        const int tile = u / nk, k0 = u - tile * nk;
+        const int ns = min(nk - k0, u1 - u);
+        u += ns;
+        const int mt = tile / cut.n_tiles, nt = tile - mt * cut.n_tiles;
+        const int m0 = mt * kTM, n0 = nt * kTN;
+        uint32_t woff[WPW], boff;
+#pragma unroll
+        for (int i = 0; i < WPW; i++) {
+            const int row = (wave * WPW + i) * 8 + (lane >> 3);
+            woff[i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + k0 * kTK + ((lane & 7) ^ (row & 7)) * 4;
+        }
+        {
+            const int row = wave * 16 + (lane >> 2);
+            boff = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
+        }
+        auto issue = [&](int st) {
+            unsigned char *dst = smem + (st % kFStages) * kFStage;
+#pragma unroll
+            for (int i = 0; i < WPW; i++)
+                __builtin_amdgcn_global_load_lds(a.Wf + woff[i] + st * kTK, dst + (wave * WPW + i) * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(a.Bhi + boff + st * kTK, dst + kFWTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(a.Blo + boff + st * kTK, dst + kFWTile + kTBTile + wave * 1024, 16, 0, 0);
+        };
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(0);
+        if (ns > 1) issue(1);
+        f32x4 acc[FI][FJ];
+#pragma unroll
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const bool live = n0 + wn * 64 < a.N && m0 + wm * 64 < a.M;
+        for (int st = 0; st < ns; st++) {
+            // step st has landed once at most the next step's DMAs are outstanding
+            if (st + 1 < ns)
+                __builtin_amdgcn_s_waitcnt(0xF70 | DPS);
+            else
+                __builtin_amdgcn_s_waitcnt(0xF70);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();  // step st - 1's reads are done in every wave
+            asm volatile("" ::: "memory");
+            if (st + 2 < ns) issue(st + 2);
+            if (!live) continue;
+            const unsigned char *sm = smem + (st % kFStages) * kFStage;
+            bf16x8 fh[FJ], fl[FJ];
+#pragma unroll
+            for (int j = 0; j < FJ; j++) {
+                fh[j] = *reinterpret_cast<const bf16x8 *>(sm + bo[j]);
+                fl[j] = *reinterpret_cast<const bf16x8 *>(sm + bo[j] + kTBTile);
+            }
+#pragma unroll
+            for (int i = 0; i < FI; i++) {
+                bf16x8 p[3];
+                split3(*reinterpret_cast<const f32x4 *>(sm + ao[i][0]), *reinterpret_cast<const f32x4 *>(sm + ao[i][1]), p);
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+#pragma unroll
+                    for (int j = 0; j < FJ; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[k], fh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < FJ; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[k], fl[j], acc[i][j], 0, 0, 0);
+                }
+            }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();  // the ring is free for the output staging
@@ -1281,7 +1374,10 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
 
 template <int EPI>
 void launch_span_epi(const GemmArgs &a, const SpanCut &cut, int tiles, int G, hipStream_t s) {
-    hipLaunchKernelGGL(gemm_span_kernel<EPI>, dim3(G), dim3(kGWaves * 64), 0, s, a, cut);
+    if (a.Wf)
+        hipLaunchKernelGGL(gemm_f32w_span_kernel<EPI>, dim3(G), dim3(kGWaves * 64), 0, s, a, cut);
+    else
+        hipLaunchKernelGGL(gemm_span_kernel<EPI>, dim3(G), dim3(kGWaves * 64), 0, s, a, cut);
     if (G != tiles) hipLaunchKernelGGL(gemm_span_reduce_kernel<EPI>, dim3(tiles * 8), dim3(kBlock), 0, s, a, cut);
 }
 
@@ -1317,10 +1413,11 @@ struct SpanPlan {
 SpanPlan plan_span(const GemmArgs &a) {
     const int tiles = ((a.M + kTM - 1) / kTM) * ((a.N + kTN - 1) / kTN), nk = a.K / kTK;
     const int64_t units = (int64_t)tiles * nk;
-    SpanPlan p{tiles, 6.0 + (double)((tiles + kSpanSlots - 1) / kSpanSlots) * nk};
+    const double step = a.Wf ? 2.0 : 1.0;  // six MFMAs instead of two, half the time in data movement
+    SpanPlan p{tiles, 6.0 + step * ((tiles + kSpanSlots - 1) / kSpanSlots) * nk};
     if (a.part)
         for (int g = 32; g <= kSpanSlots && units >= 4 * g; g += 16) {
-            const double us = 16.0 + (double)((units + g - 1) / g) + 0.06 * g;
+            const double us = 16.0 + step * (double)((units + g - 1) / g) + 0.06 * g;
             if (us < p.us) p = SpanPlan{g, us};
         }
     return p;
@@ -1377,15 +1474,7 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     if (a.Wf) {
         // f32 weights: the per-element epilogue only (no norm hand-off, no row scales)
         if (a.nrm_w || a.nss_in || a.wscale) return hipErrorInvalidValue;
-        const dim3 grid((a.M + 15) / 16, (a.N + 63) / 64);
-        switch (epi) {
-            case GEPI_STORE: hipLaunchKernelGGL(gemm_f32w_kernel<GEPI_STORE>, grid, dim3(kBlock), 0, s, a); break;
-            case GEPI_RESID: hipLaunchKernelGGL(gemm_f32w_kernel<GEPI_RESID>, grid, dim3(kBlock), 0, s, a); break;
-            case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_f32w_kernel<GEPI_SWIGLU>, grid, dim3(kBlock), 0, s, a); break;
-            case GEPI_QKV: hipLaunchKernelGGL(gemm_f32w_kernel<GEPI_QKV>, grid, dim3(kBlock), 0, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
+        return launch_span(epi, a, s);
     }
     if ((a.nrm_w || a.nss_in) && !gemm_stages_output(a.M, a.N, a.K)) return hipErrorInvalidValue;
     if (a.nrm_w && (epi != GEPI_RESID || a.M % 64 != 0 || !a.nss || !a.nx_hi || !a.nx_lo)) return hipErrorInvalidValue;
