@@ -824,7 +824,7 @@ __global__ __launch_bounds__(kBlock) void gemm_span_reduce_kernel(const GemmArgs
     f32x4 acc[4][1];
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int NC = 6;  // spans in flight
+    constexpr int NC = 3;  // spans in flight
 #pragma unroll 1
     for (int c = c0; c <= c1; c += NC) {
         f32x4 v[NC][4];
@@ -844,6 +844,107 @@ __global__ __launch_bounds__(kBlock) void gemm_span_reduce_kernel(const GemmArgs
                     for (int e = 0; e < 4; e++) acc[i][0][e] += v[x][i][e];
     }
     stage_epilogue<EPI, 4, 1, 4, true>(a, stage + wave * 16 * kStagePitch, mw, nw, acc, &pre);
+}
+
+// Tiled MFMA GEMM of 128 weight rows x 128 tokens, K in steps of 64, for grids
+// that whole tiles of this size fill (launch_gemm).
+//
+// The W / Bhi / Blo tiles go global -> LDS directly (global_load_lds_dwordx4,
+// no register staging) through a 3-stage ring, so step s + 2 is in flight
+// while step s is multiplied and each step needs one barrier.  LDS rows are unpadded 128 B with the 16-byte chunks
+// XOR-swizzled by (row & 7) against bank conflicts: a DMA wave-instruction
+// fills 1 KB = 8 rows contiguously, so each lane fetches the global chunk that
+// belongs at its LDS slot.
+constexpr int kDM = 128, kDN = 128, kDK = 64;
+constexpr int kDStages = 3;
+constexpr int kDTile = kDM * kDK * 2;  // bytes of one 128 x 64 bf16 tile
+
+// NW = 8 wavefronts (two per SIMD, so one's MFMAs overlap the other's LDS
+// reads): wave w owns rows 64 (w & 1) .. +63 and tokens 32 (w >> 1) .. +31
+// (4 x 2 MFMA fragments) and issues two of each tile's 16 DMA instructions.
+template <int EPI>
+__global__ __launch_bounds__(kGWaves * 64) void gemm_dma_kernel(const GemmArgs a) {
+    constexpr int DPW = 16 / kGWaves;  // DMA instructions per wave per tile
+    constexpr int NJ = kDN / 16 / (kGWaves / 2);  // token fragments per wave
+    static_assert(3 * DPW <= 15, "vmcnt immediate");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[kDStages * 3 * kDTile];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int wm = wave & 1, wn = wave >> 1;
+    const int m0 = blockIdx.x * kDM, n0 = blockIdx.y * kDN;
+    const int K = a.K;
+    const int nsteps = K / kDK;
+    // DMA: wave w's instruction i fills rows (DPW w + i) * 8 .. +7 of a tile;
+    // lane l writes row (DPW w + i) * 8 + (l >> 3), physical chunk l & 7, which
+    // holds logical chunk (l & 7) ^ (row & 7)
+    uint32_t off[3][DPW];
+#pragma unroll
+    for (int i = 0; i < DPW; i++) {
+        const int row = (wave * DPW + i) * 8 + (lane >> 3);
+        const int lc = (lane & 7) ^ (row & 7);
+        off[0][i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + lc * 8;
+        off[1][i] = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + lc * 8;
+        off[2][i] = off[1][i];
+    }
+    auto issue = [&](int stage, int k0) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            const uint16_t *base = x == 0 ? a.W : (x == 1 ? a.Bhi : a.Blo);
+#pragma unroll
+            for (int i = 0; i < DPW; i++)
+                __builtin_amdgcn_global_load_lds(base + off[x][i] + k0,
+                                                 smem + (stage * 3 + x) * kDTile + (wave * DPW + i) * 1024, 16, 0, 0);
+        }
+    };
+    issue(0, 0);
+    if (nsteps > 1) issue(1, kDK);
+    f32x4 acc[4][NJ];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int r = lane & 15, q4 = lane >> 4;
+    for (int st = 0; st < nsteps; st++) {
+        // this step's 3 DPW DMAs are complete once at most the next step's are
+        // outstanding (vector memory counts complete in issue order)
+        if (st + 1 < nsteps)
+            __builtin_amdgcn_s_waitcnt(0xF70 | (3 * DPW));  // vmcnt(3 DPW)
+        else
+            __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
+        __builtin_amdgcn_s_barrier();  // every wave's DMAs for this step landed; step - 1's reads are done
+        if (st + 2 < nsteps) issue((st + 2) % kDStages, (st + 2) * kDK);
+        const unsigned char *sa = smem + ((st % kDStages) * 3 + 0) * kDTile;
+        const unsigned char *sh = sa + kDTile, *sl = sa + 2 * kDTile;
+#pragma unroll
+        for (int kk = 0; kk < kDK; kk += 32) {
+            const int lc = kk / 8 + q4;
+            bf16x8 fa[4], fh[NJ], fl[NJ];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int ra = wm * 64 + i * 16 + r;
+                fa[i] = *reinterpret_cast<const bf16x8 *>(sa + ra * 128 + ((lc ^ (ra & 7)) * 16));
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const int rb = wn * NJ * 16 + j * 16 + r;
+                fh[j] = *reinterpret_cast<const bf16x8 *>(sh + rb * 128 + ((lc ^ (rb & 7)) * 16));
+                fl[j] = *reinterpret_cast<const bf16x8 *>(sl + rb * 128 + ((lc ^ (rb & 7)) * 16));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fl[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // the ring is free once every wave is past its last fragment reads
+    __builtin_amdgcn_s_barrier();
+    stage_epilogue<EPI, 4, NJ, 1>(a, reinterpret_cast<float *>(smem) + wave * NJ * 16 * kStagePitch, m0 + wm * 64,
+                               n0 + wn * NJ * 16, acc);
 }
 
 // Large-tile MFMA GEMM for long prompts: workgroup tile 256 weight rows x
@@ -1000,7 +1101,8 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_big_kernel(const GemmArgs a
                                 n0 + wn * 64, acc);
 }
 
-// Split-K MFMA GEMM for short prompts (fewer than kTiledMinTokens tokens).
+// Split-K MFMA GEMM for short prompts (up to 64 tokens; the 128-row form below up
+// to kShortMaxTokens).
 //
 // Workgroup tile: 64 weight rows x 64 tokens over one contiguous range of K
 // (split ks of nsplit).  Each 64-wide K step's W, Bhi and Blo tiles go
@@ -1381,21 +1483,27 @@ void launch_span_epi(const GemmArgs &a, const SpanCut &cut, int tiles, int G, hi
     if (G != tiles) hipLaunchKernelGGL(gemm_span_reduce_kernel<EPI>, dim3(tiles * 8), dim3(kBlock), 0, s, a, cut);
 }
 
-// Estimated microseconds of a GEMM on the three kernels that take more than
-// 64 tokens, from kernel traces of the 1B and 4B shapes at 75-8192 tokens.
-// Each is a fixed cost (launch, ring fill, epilogue) plus the K steps of the
-// longest workgroup: a 32-wide step of the 256 x 128 tile takes 0.9-1.1 us, of
-// the 256 x 256 tile 1.8, a 64-wide step of the 128 x 64 tile 0.6-0.75; a
-// K split of the short-prompt kernel costs about 5 us for its exchange, one
-// of the span kernel about 10 us plus 0.06 us per span (128 KB of partials
-// written and read back).  Choosing by them instead of by token count alone
-// (256 x 256 from 240 tiles, 128 x 128 from 256 tokens) takes the 1B prefill
-// from 6.6 to 3.95 ms at 301 tokens, 7.0 to 4.5 at 500, 8.3 to 7.3 at 1000,
-// 11.9 to 10.9 at 1500 and 20.7 to 19.0 at 3001, and leaves 100, 2000, 4096
-// and 8192 as they were.
+// Estimated microseconds of a GEMM on the four kernels that take more than 64
+// tokens, from kernel traces of the 1B and 4B shapes at 75-8192 tokens.  Each
+// is a fixed cost (launch, ring fill, epilogue) plus the K steps of the
+// longest workgroup: a 64-wide step of the 128 x 128 tile takes 1.02 us, 1.2
+// where several rounds keep the chip full; a 32-wide step of the 256 x 128
+// tile 1.1 us (0.95 in one round of whole tiles), of the 256 x 256 tile 1.8; a 64-wide step of the 128 x 64 tile
+// 0.6-0.75.  A K split of the short-prompt kernel costs about 5 us for its
+// exchange, one of the span kernel about 8 us plus 0.06 us per span (128 KB of
+// partials written and read back).  Choosing by them instead of by token count
+// (256 x 256 from 240 tiles, 128 x 128 from 256 tokens) and with the span
+// kernel, the 1B prefill went from 6.6 to 3.95 ms at 301 tokens, 7.0 to 4.5 at
+// 500, 11.9 to 10.9 at 1500, the 4B prefill from 14.5 to 7.7 at 300 and 18.0
+// to 15.9 at 700.
 double big_us(const GemmArgs &a) {
     const int wg = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
     return 8.0 + 1.8 * ((wg + 255) / 256) * (a.K / kBK);
+}
+
+double dma_us(const GemmArgs &a) {
+    const int wg = ((a.M + kDM - 1) / kDM) * ((a.N + kDN - 1) / kDN);
+    return 6.0 + (wg <= 256 ? 1.02 : 1.2) * ((wg + 255) / 256) * (a.K / kDK);
 }
 
 double skinny_wide_us(const GemmArgs &a) {
@@ -1413,11 +1521,13 @@ struct SpanPlan {
 SpanPlan plan_span(const GemmArgs &a) {
     const int tiles = ((a.M + kTM - 1) / kTM) * ((a.N + kTN - 1) / kTN), nk = a.K / kTK;
     const int64_t units = (int64_t)tiles * nk;
-    const double step = a.Wf ? 2.0 : 1.0;  // six MFMAs instead of two, half the time in data movement
-    SpanPlan p{tiles, 6.0 + step * ((tiles + kSpanSlots - 1) / kSpanSlots) * nk};
+    // f32 weights: six MFMAs instead of two, half the time in data movement
+    const double kind = a.Wf ? 2.0 : 1.0, step = 1.1 * kind;
+    const int rounds = (tiles + kSpanSlots - 1) / kSpanSlots;
+    SpanPlan p{tiles, 6.0 + (rounds > 1 ? step : 0.95 * kind) * rounds * nk};
     if (a.part)
         for (int g = 32; g <= kSpanSlots && units >= 4 * g; g += 16) {
-            const double us = 16.0 + step * (double)((units + g - 1) / g) + 0.06 * g;
+            const double us = 14.0 + step * (double)((units + g - 1) / g) + 0.06 * g;
             if (us < p.us) p = SpanPlan{g, us};
         }
     return p;
@@ -1482,13 +1592,24 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     const bool tiled = a.K % 64 == 0 && a.N > 64;
     const double span_us = tiled ? plan_span(a).us : HUGE_VAL;
     const double short_us = tiled && a.N <= kShortMaxTokens ? skinny_wide_us(a) : HUGE_VAL;
-    if (a.N >= kTiledMinTokens && (tiled ? big_us(a) < std::min(span_us, short_us) : big_fills(a.M, a.N))) {
+    if (a.N >= kTiledMinTokens && (tiled ? big_us(a) < std::min({span_us, short_us, dma_us(a)}) : big_fills(a.M, a.N))) {
         const dim3 grid((a.M + kBM - 1) / kBM, (a.N + kBN - 1) / kBN);
         switch (epi) {
             case GEPI_STORE: hipLaunchKernelGGL(gemm_big_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
             case GEPI_RESID: hipLaunchKernelGGL(gemm_big_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
             case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_big_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
             case GEPI_QKV: hipLaunchKernelGGL(gemm_big_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
+            default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    }
+    if (tiled && a.N >= kTiledMinTokens && dma_us(a) < std::min(span_us, short_us)) {
+        const dim3 grid((a.M + kDM - 1) / kDM, (a.N + kDN - 1) / kDN);
+        switch (epi) {
+            case GEPI_STORE: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
+            case GEPI_RESID: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
+            case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
+            case GEPI_QKV: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
             default: return hipErrorInvalidValue;
         }
         return hipGetLastError();
