@@ -33,6 +33,15 @@ _open = {}
 def _models(mods, which):
     if which not in _open:
         T, O, W = mods
+        if which.startswith("i8-"):
+            wl = _models(mods, which[3:])[2]
+            p = W.ensure_model(wl, model_root())
+            os.environ["TMG_I8"] = "1"
+            try:
+                _open[which] = T.Model.load(p), O.OracleModel.load(p, i8=True), wl
+            finally:
+                del os.environ["TMG_I8"]
+            return _open[which]
         if which.startswith("f32-"):
             from f32models import variant
             wl = _models(mods, which[4:])[2]
@@ -104,3 +113,47 @@ def test_attention_key_runs(mods, which, pieces):
                                           ("f32-h1088", [2, 255]), ("f32-h1088", [300])])
 def test_f32_weight_gemm(mods, which, pieces):
     _check(mods, which, pieces)
+
+
+# int8 codes: the row scales in the epilogues of whole and of split tiles
+@pytest.mark.parametrize("n", [130, 577, 1025])
+def test_i8_spans(mods, n):
+    _check(mods, "i8-1b", [n])
+
+
+def test_rows_before_a_non_finite_one(mods):
+    # a token whose embedding is infinite makes its own row NaN and no earlier
+    # one: its keys and values are masked for them, whose attention must not
+    # meet 0 * NaN (the fp32 kernel's key-by-key block)
+    import shutil
+
+    from f32models import write_safetensors
+    T, O, W = mods
+    wl = dataclasses.replace(W.ONE_B, name="minicpm5-1b-synthetic-l2-v512", num_hidden_layers=2, vocab_size=512,
+                             weight_seed=31)
+    src = W.ensure_model(wl, model_root())
+    d = os.path.join(model_root(), wl.name + "-inf-row")
+    path = os.path.join(d, "model.safetensors")
+    if not os.path.exists(path):
+        os.makedirs(d, exist_ok=True)
+        tensors = {}
+        for name, t in O.load_safetensors(src).items():
+            data = np.array(t.data)
+            if name == "model.embed_tokens.weight":
+                data.reshape(wl.vocab_size, -1)[7] = 0x7F80
+            tensors[name] = (t.dtype, t.shape, data.tobytes())
+        shutil.copy(os.path.join(os.path.dirname(src), "config.json"), os.path.join(d, "config.json"))
+        write_safetensors(path, tensors)
+    g = T.Model.load(path)
+    ids = [8 + int(t) % 500 for t in T.synth_tokens(89, 1064, wl.vocab_size)]
+    kv = []
+    for last in (ids[-1], 7):
+        c = T.KvCache(g, 1064)
+        g.forward_seq(ids[:1000], c)
+        g.forward_seq(ids[1000:1063] + [last], c)
+        kv.append((c.keys_flat(1).reshape(1064, -1)[:1063], c.values_flat(1).reshape(1064, -1)[:1063]))
+        c.close()
+    for a, b in zip(*kv):
+        assert np.all(np.isfinite(b))
+        _close(b, a, "rows before the NaN one")
+    g.close()

@@ -117,8 +117,8 @@ namespace tmg {
 // ceil(max_pos / attn_block) splits (at most kMaxSplits).  Up to kFusedSplits
 // the merge runs in the o_proj prologue, above in attn_combine_kernel.
 constexpr int kMaxSplits = 32;
-// Sequences per tmg_generate_batch call (the short-prompt GEMM takes up to
-// 255 token rows; the bound keeps the per-call KV allocation in view).
+// Sequences per tmg_generate_batch call (the bound keeps the per-call KV
+// allocation in view).
 constexpr int kMaxBatch = 128;
 
 // Launch filter used by tmg_profile_decode_step: every kernel of the step is
