@@ -92,3 +92,29 @@ def variant(src_path, dst_root, kind, seed=7):
     write_safetensors(out, tensors)
     shutil.copy(os.path.join(os.path.dirname(src_path), "config.json"), os.path.join(d, "config.json"))
     return out
+
+
+def edited(src_path, dst_root, name, edit):
+    """The model at src_path with edit(tensor name, array) -> the array to
+    store in its place (BF16 as uint16, F16 / F32 as such; None keeps what it
+    was given, changed or not), as <dst_root>/<name>/model.safetensors."""
+    d = os.path.join(dst_root, name)
+    out = os.path.join(d, "model.safetensors")
+    if os.path.exists(out):
+        return out
+    os.makedirs(d, exist_ok=True)
+    kinds = {"BF16": np.uint16, "F16": np.float16, "F32": np.float32}
+    with open(src_path, "rb") as f:
+        raw = f.read()
+    n = struct.unpack("<Q", raw[:8])[0]
+    tensors = {}
+    for tname, e in json.loads(raw[8:8 + n]).items():
+        if tname == "__metadata__":
+            continue
+        a, b = e["data_offsets"]
+        data = np.frombuffer(raw[8 + n + a:8 + n + b], kinds[e["dtype"]]).reshape(e["shape"]).copy()
+        new = edit(tname, data)
+        tensors[tname] = (e["dtype"], e["shape"], (data if new is None else new).tobytes())
+    shutil.copy(os.path.join(os.path.dirname(src_path), "config.json"), os.path.join(d, "config.json"))
+    write_safetensors(out, tensors)
+    return out

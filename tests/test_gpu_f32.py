@@ -5,12 +5,13 @@ MFMA prefill GEMM and the loader, against the oracle's f32 path on the same
 files.  Tolerances are the decode path's (logits within 2e-3 abs + 1e-3 rel,
 greedy ids identical)."""
 import dataclasses
+import os
 
 import numpy as np
 import pytest
 
 from conftest import model_root
-from f32models import variant
+from f32models import edited, variant
 
 pytestmark = pytest.mark.gpu
 
@@ -159,3 +160,43 @@ def test_batch_rejects_f32_models(T, untied_path):
     g = T.Model.load(variant(untied_path, model_root(), "f32"))
     with pytest.raises(T.TmgError, match="f32 weight matrices"):
         T.generate_batch(g, [[1, 2], [3]], 4)
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16"])
+def test_prefill_non_finite_weight(T, O, untied_path, kind):
+    # an infinite weight times an activation x is x's sign of infinity, alone
+    # and beside finite products, and a NaN stays one whatever its payload:
+    # the rows that hold them, in prefill as in the one-token GEMV, at K steps
+    # in the middle and at the end
+    src = variant(untied_path, model_root(), kind)
+
+    def edit(name, w):
+        if name == "model.layers.0.self_attn.v_proj.weight":
+            w[3, 5] = np.inf
+            w[4, -1] = -np.inf
+            if kind == "f32":
+                w.view(np.uint32)[9, 7] = 0x7F800001  # payload in the low 16 bits only
+            else:
+                w.view(np.uint16)[9, 7] = 0x7C01
+        if name == "model.layers.0.self_attn.k_proj.weight":
+            w[2, 11] = np.inf
+
+    path = edited(src, model_root(), f"{os.path.basename(os.path.dirname(src))}-nonfinite", edit)
+    g, o = T.Model.load(path), O.OracleModel.load(path)
+    for n in (1, 20, 200):
+        print(f"non-finite {kind} weights, {n} tokens", flush=True)
+        ids = [int(t) for t in T.synth_tokens(37, n + 1, g.config.vocab_size)]
+        gc, oc = T.KvCache(g, n + 8), o.new_cache()
+        g.forward_seq(ids[:n], gc)
+        o.forward_seq(ids[:n], oc)
+        g.forward_token(ids[n], gc)
+        o.forward_token(ids[n], oc)
+        for a, b in ((gc.keys_flat(0), oc.keys_flat(0)), (gc.values_flat(0), oc.values_flat(0))):
+            a, b = np.asarray(a), np.asarray(b)
+            assert np.isinf(b).any() or np.isnan(b).any()
+            assert np.array_equal(np.isnan(a), np.isnan(b))
+            assert np.array_equal(a[np.isinf(b)], b[np.isinf(b)])
+            fin = np.isfinite(b)
+            assert np.all(np.isfinite(a[fin])) and np.abs(a[fin] - b[fin]).max() < 1e-4
+        gc.close()
+    g.close()

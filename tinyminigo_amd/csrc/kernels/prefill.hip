@@ -657,16 +657,16 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_span_kernel(const GemmArgs 
     }
 }
 
-// Eight f32 weights of a row as three bf16 parts that sum to them exactly:
-// the upper 8 significand bits by truncation, twice, and the rest.
+// Eight f32 weights of a row as three bf16 parts that sum to them exactly: the
+// upper 8 significand bits by truncation, twice, and the rest.  The second and
+// third part of an infinite or NaN weight are NaN.
 __device__ __forceinline__ void split3(const f32x4 &x0, const f32x4 &x1, bf16x8 (&p)[3]) {
     uint32_t b[3][8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const float x = i < 4 ? x0[i & 3] : x1[i & 3];
         b[0][i] = __float_as_uint(x) & 0xffff0000u;
-        // an infinity is its first part alone (inf - inf is NaN)
-        const float r = fabsf(x) < INFINITY ? x - __uint_as_float(b[0][i]) : 0.0f;
+        const float r = x - __uint_as_float(b[0][i]);
         b[1][i] = __float_as_uint(r) & 0xffff0000u;
         b[2][i] = __float_as_uint(r - __uint_as_float(b[1][i]));
     }
@@ -679,6 +679,42 @@ __device__ __forceinline__ void split3(const f32x4 &x0, const f32x4 &x1, bf16x8 
     }
 }
 
+// One wavefront's 64 x 64 outputs over `ns` K steps from step k0 as
+// gemm_f32w_span_kernel's, on the fp32 MFMA from memory: each weight times
+// hi + lo.  Lane (r, q4) holds k 8 q4 .. +7 of its rows and tokens, and MFMA e
+// takes the e-th of them from every lane.
+__device__ __forceinline__ void f32w_tile(const GemmArgs &a, int mw, int nw, int k0, int ns, f32x4 (&acc)[4][4]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
+    const float *w[4];
+    const uint16_t *h[4], *l[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const size_t at = (size_t)k0 * kTK + 8 * q4;
+        w[i] = a.Wf + (size_t)min(mw + i * 16 + r, a.M - 1) * a.K + at;
+        const size_t n = (size_t)min(nw + i * 16 + r, a.N - 1) * a.K + at;
+        h[i] = a.Bhi + n;
+        l[i] = a.Blo + n;
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll 1
+    for (int k = 0; k < ns * kTK; k += kTK) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float x[4], y[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                x[i] = w[i][k + e];
+                y[i] = bf16_to_f32(h[i][k + e]) + bf16_to_f32(l[i][k + e]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[j], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
 // gemm_span_kernel over f32 weights (WMat::F32; matmul_batch_w_into's F32
 // arm, src/tensor.rs:573-760): the W tile is staged as f32 (128-byte rows,
 // chunks XOR-swizzled by row & 7, three 48 KB stages) and each fragment is
@@ -686,8 +722,10 @@ __device__ __forceinline__ void split3(const f32x4 &x0, const f32x4 &x1, bf16x8 
 // exact products of f32 weights and hi + lo activations: at 16 times the fp32
 // MFMA's rate, still faster than its four per 16 k.  It replaced an unstaged
 // 16 x 64 kernel on the fp32 MFMA, bound by L2 reads of its operands: four 1B
-// layers of F16 weights 1.20 -> 0.65 ms at 2 tokens, 1.69 -> 0.72 at 64, 3.48
-// -> 1.17 at 200, 14.2 -> 2.9 at 1000.
+// layers of F16 weights 1.20 -> 0.66 ms at 2 tokens, 1.69 -> 0.74 at 64, 3.48
+// -> 1.16 at 200, 14.2 -> 2.8 at 1000.  An infinite or NaN weight leaves NaN in
+// its row's outputs (its parts meet as inf - inf); a wavefront with NaN outputs
+// computes them again from the whole weights (f32w_tile).
 constexpr int kFWTile = kTM * kTK * 4, kFStage = kFWTile + 2 * kTBTile, kFStages = 3;
 
 template <int EPI>
@@ -790,6 +828,14 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_f32w_span_kernel(const Gemm
         __builtin_amdgcn_s_barrier();  // the ring is free for the output staging
         asm volatile("" ::: "memory");
         if (!live) continue;
+        bool nan = false;
+#pragma unroll
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) nan = nan || acc[i][j][e] != acc[i][j][e];
+        if (__builtin_amdgcn_ballot_w64(nan)) f32w_tile(a, m0 + wm * 64, n0 + wn * 64, k0, ns, acc);
         if (ns < nk) {
             f32x4 *part = reinterpret_cast<f32x4 *>(a.part) +
                           (cut.slot(g, tile * nk) * kGWaves + wave) * (FI * FJ * 64) + lane;
