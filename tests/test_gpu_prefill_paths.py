@@ -157,3 +157,37 @@ def test_rows_before_a_non_finite_one(mods):
         assert np.all(np.isfinite(b))
         _close(b, a, "rows before the NaN one")
     g.close()
+
+
+def _non_finite_model(mods):
+    """Two layers; token 7's embedding is infinite, so its rows are NaN from
+    the first norm on."""
+    from f32models import edited
+    T, O, W = mods
+    wl = dataclasses.replace(W.ONE_B, name="minicpm5-1b-synthetic-l2-v512", num_hidden_layers=2, vocab_size=512,
+                             weight_seed=31)
+
+    def edit(name, w):
+        if name == "model.embed_tokens.weight":
+            w[7] = 0x7F80
+
+    return edited(W.ensure_model(wl, model_root()), model_root(), wl.name + "-inf-row", edit)
+
+
+@pytest.mark.parametrize("piece", [64, 300])
+def test_rows_after_a_run_of_non_finite_ones(mods, piece):
+    # 256 tokens whose keys and values are all NaN: a run of key blocks may
+    # hold nothing else, and its NaN has to reach every later row all the same
+    T, O, W = mods
+    g = T.Model.load(_non_finite_model(mods))
+    ids = [8 + int(t) % 500 for t in T.synth_tokens(97, 640 + piece, 512)]
+    ids[256:512] = [7] * 256
+    c = T.KvCache(g, len(ids))
+    print(f"after NaN rows: {piece}", flush=True)
+    g.forward_seq(ids[:640], c)
+    g.forward_seq(ids[640:], c)
+    k, v = c.keys_flat(1).reshape(len(ids), -1), c.values_flat(1).reshape(len(ids), -1)
+    assert np.all(np.isfinite(k[:256])) and np.all(np.isfinite(v[:256]))
+    assert np.all(np.isnan(k[256:])) and np.all(np.isnan(v[256:]))
+    c.close()
+    g.close()

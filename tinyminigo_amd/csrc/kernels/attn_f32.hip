@@ -253,7 +253,9 @@ __global__ __launch_bounds__(kBlock) void attn_f32_combine_kernel(const AttnArgs
             }
 #pragma unroll
         for (int x = 0; x < NC; x++)
-            if (s + x < nsp && ml[x].x != -INFINITY) {
+            // a run without a visible key adds nothing; one whose scores are all
+            // NaN has no maximum either, but a NaN sum, which has to go through
+            if (s + x < nsp && !(ml[x].x == -INFINITY && ml[x].y == 0.0f)) {
                 const float nm = fmaxf(M, ml[x].x);
                 const float f0 = __builtin_amdgcn_exp2f(M - nm), f1 = __builtin_amdgcn_exp2f(ml[x].x - nm);
                 M = nm;
