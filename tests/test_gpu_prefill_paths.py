@@ -191,3 +191,45 @@ def test_rows_after_a_run_of_non_finite_ones(mods, piece):
     assert np.all(np.isnan(k[256:])) and np.all(np.isnan(v[256:]))
     c.close()
     g.close()
+
+
+@pytest.mark.parametrize("pieces", [(1024, 64), (1024, 300)])
+def test_first_keys_at_minus_infinity(mods, pieces):
+    # 512 tokens whose keys score -inf against every other query (their q . k
+    # overflows): the first runs of key blocks hold no weight, the later ones
+    # all of it
+    from f32models import edited
+    T, O, W = mods
+    wl = dataclasses.replace(W.ONE_B, name="minicpm5-1b-synthetic-l1-v512-s37", num_hidden_layers=1, vocab_size=512,
+                             weight_seed=37)
+    hd, slow = wl.head_dim, wl.head_dim // 2 - 1  # the slowest RoPE pair's first dim
+
+    def bf16(x):
+        return np.float32(x).view(np.uint32) >> 16
+
+    def edit(name, w):
+        if name == "model.embed_tokens.weight":
+            w[:, :2] = 0
+            w[:8, 0] = bf16(1.0)  # tokens 0-7: these keys
+            w[8:, 1] = bf16(1.0)  # the others: their queries
+        elif name.endswith("k_proj.weight"):
+            w[slow::hd] = 0
+            w[slow::hd, 0] = bf16(-5e36)
+        elif name.endswith("q_proj.weight"):
+            w[slow::hd] = 0
+            w[slow::hd, 1] = bf16(4.0)
+
+    p = edited(W.ensure_model(wl, model_root()), model_root(), wl.name + "-minus-inf", edit)
+    g, o = T.Model.load(p), O.OracleModel.load(p)
+    n = sum(pieces)
+    ids = [8 + int(t) % 500 for t in T.synth_tokens(101, n, 512)]
+    ids[:512] = [int(t) % 8 for t in T.synth_tokens(103, 512, 512)]
+    gc, oc, at = T.KvCache(g, n), o.new_cache(), 0
+    for m in pieces:
+        print(f"first keys at -inf: {m} at {at}", flush=True)
+        a, b = g.forward_seq(ids[at:at + m], gc), o.forward_seq(ids[at:at + m], oc)
+        assert np.all(np.isfinite(b))
+        _close(a, b, f"piece of {m} at {at}")
+        at += m
+    gc.close()
+    g.close()

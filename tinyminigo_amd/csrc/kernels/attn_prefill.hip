@@ -496,8 +496,9 @@ __global__ __launch_bounds__(kBlock) void attn_prefill_combine_kernel(const Attn
             }
 #pragma unroll
         for (int x = 0; x < NC; x++)
-            if (s + x < nsp) {
-                // the first run holds key 0, so M is finite from then on
+            // a run that gives a row no weight (its keys lie past the row or
+            // score -inf) has no maximum and a zero sum; a NaN sum goes through
+            if (s + x < nsp && !(ml[x].x == -INFINITY && ml[x].y == 0.0f)) {
                 const float nm = fmaxf(M, ml[x].x);
                 const float f0 = __builtin_amdgcn_exp2f(M - nm), f1 = __builtin_amdgcn_exp2f(ml[x].x - nm);
                 M = nm;
