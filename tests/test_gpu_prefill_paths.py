@@ -174,6 +174,29 @@ def _non_finite_model(mods):
     return edited(W.ensure_model(wl, model_root()), model_root(), wl.name + "-inf-row", edit)
 
 
+# pieces that take the split-bf16 kernel, with key runs and in whole query
+# blocks (as many workgroups as the chip has CUs)
+@pytest.mark.parametrize("pieces", [(700, 300), (2112,), (256, 257)])
+def test_rows_before_a_non_finite_one_in_a_long_piece(mods, pieces):
+    T, O, W = mods
+    g = T.Model.load(_non_finite_model(mods))
+    n = sum(pieces)
+    ids = [8 + int(t) % 500 for t in T.synth_tokens(89, n, 512)]
+    kv = []
+    for last in (ids[-1], 7):
+        c, at = T.KvCache(g, n), 0
+        for p in pieces:
+            print(f"rows before token {last}: {p} at {at}", flush=True)
+            g.forward_seq((ids[:-1] + [last])[at:at + p], c)
+            at += p
+        kv.append((c.keys_flat(1).reshape(n, -1), c.values_flat(1).reshape(n, -1)))
+        c.close()
+    for a, b in zip(*kv):
+        assert np.all(np.isnan(b[-1])) and np.all(np.isfinite(b[:-1]))
+        _close(b[:-1], a[:-1], "rows before the NaN one")
+    g.close()
+
+
 @pytest.mark.parametrize("piece", [64, 300])
 def test_rows_after_a_run_of_non_finite_ones(mods, piece):
     # 256 tokens whose keys and values are all NaN: a run of key blocks may

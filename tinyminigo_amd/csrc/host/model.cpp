@@ -682,7 +682,7 @@ static int ensure_kv_split(tmg_model *m, int n) {
     int rc;
     const size_t sz = (size_t)cap * m->kvd;
     if ((rc = dev_alloc(m, &m->pf_kh, sz)) || (rc = dev_alloc(m, &m->pf_kl, sz)) || (rc = dev_alloc(m, &m->pf_vth, sz)) ||
-        (rc = dev_alloc(m, &m->pf_vtl, sz)))
+        (rc = dev_alloc(m, &m->pf_vtl, sz)) || (rc = dev_alloc(m, &m->pf_vodd, (size_t)(cap / 64 + 3) / 4 * 4 * m->nkv)))
         return rc;
     m->kv_cap = cap;
     return TMG_OK;
@@ -789,13 +789,15 @@ static int prefill_layers(tmg_model *m, int T, int start, float *k, float *v, ui
             TMG_HIP(launch_attn(aa, s));
         } else if (attn_prefill_supported(aa)) {
             if ((rc = ensure_kv_split(m, start + T))) return rc;
-            KVSplitArgs ka{kc, vc, start + T, m->nkv, m->hd, m->pf_kh, m->pf_kl, m->pf_vth, m->pf_vtl, m->kv_cap};
+            KVSplitArgs ka{kc, vc, start + T, m->nkv, m->hd, m->pf_kh, m->pf_kl, m->pf_vth, m->pf_vtl, m->kv_cap,
+                           m->pf_vodd};
             TMG_HIP(launch_kv_split(ka, s));
             aa.kh = m->pf_kh;
             aa.kl = m->pf_kl;
             aa.vth = m->pf_vth;
             aa.vtl = m->pf_vtl;
             aa.vt_pitch = m->kv_cap;
+            aa.v_odd = m->pf_vodd;
             TMG_HIP(launch_attn_prefill(aa, s));
         } else if (attn_f32_pays(aa)) {
             TMG_HIP(launch_attn_f32(aa, s));

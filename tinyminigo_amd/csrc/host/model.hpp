@@ -67,6 +67,7 @@ struct tmg_model {
     // split-bf16 KV rows for the MFMA prefill attention (rows [0, kv_cap))
     int kv_cap = 0;
     uint16_t *pf_kh = nullptr, *pf_kl = nullptr, *pf_vth = nullptr, *pf_vtl = nullptr;
+    uint8_t *pf_vodd = nullptr;  // per 64-key block and KV head: infinite or NaN values
 
     // pinned host staging
     void *pin = nullptr;

@@ -99,14 +99,22 @@ __host__ __device__ constexpr int vt_slot(int row) {
     return (row & 32) | (((row & 15) >> 2) << 3) | ((row & 16) >> 2) | (row & 3);
 }
 
+// Bytes of a head's v_odd, whole dwords.
+__host__ __device__ inline int odd_pitch(int vt_pitch) { return (vt_pitch / kPKB + 3) / 4 * 4; }
+
+// A value that bf16 cannot hold: infinite, NaN or rounded to infinity.
+__device__ __forceinline__ bool odd_value(float v) { return (f32_to_bf16_rne(v) & 0x7f80) == 0x7f80; }
+
 // One workgroup per (64 positions, KV head): f32 K/V rows -> split-bf16 K
 // [pos][kvd] and V^T [head][dim][slot] (through an LDS transpose; the keys of
-// each 64-key block in vt_slot order); rows at or past n are zeros.
+// each 64-key block in vt_slot order); rows at or past n are zeros.  Odd
+// values are zeros in V^T, and v_odd says whether the block holds one.
 __global__ __launch_bounds__(kBlock) void kv_split_kernel(const KVSplitArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t sT[2][kPHD][kSVP];
     const int t = threadIdx.x;
     const int p0 = blockIdx.x * kPKB, g = blockIdx.y;
     const int kvd = a.nkv * kPHD;
+    bool odd = false;
     // K: 64 rows x 128 dims of head g, 4 floats per thread per step
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -124,7 +132,9 @@ __global__ __launch_bounds__(kBlock) void kv_split_kernel(const KVSplitArgs a) {
         for (int j = 0; j < 4; j++) {
             split2(kk[j], kh[j], kl[j]);
             uint16_t vh, vl;
-            split2(vv[j], vh, vl);
+            const bool o = odd_value(vv[j]);
+            odd = odd || o;
+            split2(o ? 0.0f : vv[j], vh, vl);
             sT[0][d + j][prow] = vh;
             sT[1][d + j][prow] = vl;
         }
@@ -134,7 +144,8 @@ __global__ __launch_bounds__(kBlock) void kv_split_kernel(const KVSplitArgs a) {
         *reinterpret_cast<u32x2 *>(a.kl + o) =
             u32x2{(uint32_t)kl[0] | ((uint32_t)kl[1] << 16), (uint32_t)kl[2] | ((uint32_t)kl[3] << 16)};
     }
-    __syncthreads();
+    odd = __syncthreads_or(odd);
+    if (t == 0) a.v_odd[(size_t)g * odd_pitch(a.vt_pitch) + blockIdx.x] = odd;
     // V^T: 128 dim rows x 64 positions, 16 bytes per thread per step
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -221,6 +232,12 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
 #pragma unroll
     for (int qt = 0; qt < kPQT; qt++) live = live || __builtin_amdgcn_ballot_w64(ti[qt] < a.T) != 0;
 
+    // whether a block near the run holds odd values: four per load, the first
+    // 256 in flight with Q
+    const uint8_t *const v_odd = a.v_odd + (size_t)g * odd_pitch(a.vt_pitch);
+    uint32_t odd = 0;
+    if ((kb0 / 4 + lane) * 4 < kb1) odd = *reinterpret_cast<const uint32_t *>(v_odd + 4 * (kb0 / 4 + lane));
+
     // Q is pre-scaled by scale / ln 2, so the scores come out in log2 units
     const float sl2 = a.scale * 1.4426950408889634f;
     // Q^T fragments (MFMA B operand): dims 32 ds + 8 q4 .. +7 of the column.
@@ -239,6 +256,7 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
             split8(v, qh[qt][ds], ql[qt][ds]);
         }
     }
+    for (int b = kb0 / 4 + 64 + lane; b * 4 < kb1; b += 64) odd |= *reinterpret_cast<const uint32_t *>(v_odd + 4 * b);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // DMA map: wave w's instruction i fills 1 KB slice 2 w + (i & 1) of part
@@ -437,6 +455,38 @@ __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnAr
     }
     if (kb < kb1) iteration(kb, sc[0], sc[1]);
     if (!live) return;
+    // the products of the odd values, left out so far (zero times such a value
+    // of a masked key would not be zero): key by key, each lane a quarter of
+    // its column's score.  Behind the loop: within it, in the diagonal blocks,
+    // this code cost the 8192-token prefill 1.3%; here nothing measurable
+    if (__builtin_amdgcn_ballot_w64(odd != 0)) {
+#pragma unroll 1
+        for (int key = kb0 * kPKB; key < min(kb1 * kPKB, a.start + a.T); key++) {
+            if (!v_odd[key / kPKB]) {
+                key |= kPKB - 1;
+                continue;
+            }
+            const float *krow = a.k_cache + (size_t)key * kvd + g * kPHD + 32 * q4;
+            const float *vrow = a.v_cache + (size_t)key * kvd + g * kPHD + 4 * q4;
+#pragma unroll
+            for (int qt = 0; qt < kPQT; qt++) {
+                const float *qrow = a.q + (size_t)min(ti[qt], a.T - 1) * qd + qhead[qt] * kPHD + 32 * q4;
+                float s = 0.0f;
+#pragma unroll 4
+                for (int d = 0; d < 32; d++) s += qrow[d] * krow[d];
+                s = add_xor32(add_xor16(s)) * sl2;
+                if (key > qpos[qt]) continue;
+                const float p = __builtin_amdgcn_exp2f(s - (m[qt] == -INFINITY ? 0.0f : m[qt]));
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(vrow + 16 * dt);
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (odd_value(v[i])) o[qt][dt][i] += p * v[i];
+                }
+            }
+        }
+    }
     // normalize and write the split-bf16 output (O^T rows dims 16 dt + 4 q4 +
     // i), or with several runs the unnormalized output, maximum and sum
 #pragma unroll
@@ -522,7 +572,7 @@ __global__ __launch_bounds__(kBlock) void attn_prefill_combine_kernel(const Attn
 }  // namespace
 
 hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s) {
-    if (a.hd != kPHD || a.n <= 0 || a.vt_pitch < (a.n + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)
+    if (a.hd != kPHD || a.n <= 0 || !a.v_odd || a.vt_pitch < (a.n + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(kv_split_kernel, dim3((a.n + kPKB - 1) / kPKB, a.nkv), dim3(kBlock), 0, s, a);
     return hipGetLastError();
@@ -592,7 +642,7 @@ bool attn_prefill_supported(const AttnArgs &a) {
 
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s) {
     if (!attn_prefill_supported(a) || a.T <= 0 || !a.kh || !a.kl || !a.vth || !a.vtl ||
-        a.vt_pitch < (a.start + a.T + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)
+        !a.v_odd || !a.k_cache || !a.v_cache || a.vt_pitch < (a.start + a.T + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)
         return hipErrorInvalidValue;
     switch (a.nq / a.nkv) {
         case 1: launch_attn_prefill_group<1>(a, s); break;

@@ -130,19 +130,22 @@ struct AttnArgs {
     // [pos][nkv*hd] and values transposed [nkv][hd][vt_pitch]
     const uint16_t *kh, *kl, *vth, *vtl;
     int vt_pitch;
+    const uint8_t *v_odd;  // [nkv][64-key block]: it holds values that bf16 cannot, zeros in vth / vtl
     // set by launch_attn_prefill: most key blocks per workgroup (0: all); part
     // and part_ml then hold the runs of up to kAttnRuns workgroups
     int key_run;
 };
 
 // Split-bf16 copies of one layer's KV cache rows [0, n) for the MFMA prefill
-// attention (rows up to the next multiple of 64 are zeros).
+// attention (rows up to the next multiple of 64 are zeros), and which 64-key
+// blocks hold infinite or NaN values.
 struct KVSplitArgs {
     const float *k_cache, *v_cache;  // [pos][nkv*hd]
     int n, nkv, hd;
     uint16_t *kh, *kl;               // [round64(n)][nkv*hd]
     uint16_t *vth, *vtl;             // [nkv][hd][vt_pitch], vt_pitch >= round64(n)
     int vt_pitch;
+    uint8_t *v_odd;                  // [nkv][vt_pitch / 64 rounded up to a multiple of 4]
 };
 hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s);
 
