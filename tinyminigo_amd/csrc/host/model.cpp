@@ -682,7 +682,7 @@ static int ensure_kv_split(tmg_model *m, int n) {
     int rc;
     const size_t sz = (size_t)cap * m->kvd;
     if ((rc = dev_alloc(m, &m->pf_kh, sz)) || (rc = dev_alloc(m, &m->pf_kl, sz)) || (rc = dev_alloc(m, &m->pf_vth, sz)) ||
-        (rc = dev_alloc(m, &m->pf_vtl, sz)) || (rc = dev_alloc(m, &m->pf_vodd, (size_t)(cap / 64 + 3) / 4 * 4 * m->nkv)))
+        (rc = dev_alloc(m, &m->pf_vtl, sz)) || (rc = dev_alloc(m, &m->pf_vodd, (size_t)(cap / 64 + 3) / 4 * 16 * m->nkv)))
         return rc;
     m->kv_cap = cap;
     return TMG_OK;

@@ -130,7 +130,7 @@ struct AttnArgs {
     // [pos][nkv*hd] and values transposed [nkv][hd][vt_pitch]
     const uint16_t *kh, *kl, *vth, *vtl;
     int vt_pitch;
-    const uint8_t *v_odd;  // [nkv][64-key block]: it holds values that bf16 cannot, zeros in vth / vtl
+    const uint8_t *v_odd;  // [nkv][64-key block][4]: it holds values that bf16 cannot, zeros in vth / vtl
     // set by launch_attn_prefill: most key blocks per workgroup (0: all); part
     // and part_ml then hold the runs of up to kAttnRuns workgroups
     int key_run;
@@ -145,7 +145,7 @@ struct KVSplitArgs {
     uint16_t *kh, *kl;               // [round64(n)][nkv*hd]
     uint16_t *vth, *vtl;             // [nkv][hd][vt_pitch], vt_pitch >= round64(n)
     int vt_pitch;
-    uint8_t *v_odd;                  // [nkv][vt_pitch / 64 rounded up to a multiple of 4]
+    uint8_t *v_odd;                  // [nkv][vt_pitch / 64 rounded up to a multiple of 4][4], 16-byte aligned
 };
 hipError_t launch_kv_split(const KVSplitArgs &a, hipStream_t s);
 
