@@ -200,3 +200,28 @@ def test_prefill_non_finite_weight(T, O, untied_path, kind):
             assert np.all(np.isfinite(a[fin])) and np.abs(a[fin] - b[fin]).max() < 1e-4
         gc.close()
     g.close()
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_operand_of_more_than_2_32_elements(T, W, kind):
+    # intermediate 16384 and 262208 tokens: the last 64 rows of the down
+    # projection's operand lie past 2^32 elements.  The call against the same
+    # ids in two, whose second takes those rows as an operand of its own
+    wl = dataclasses.replace(W.TINY, name="llama-h128-i16384-l1", hidden_size=128, num_hidden_layers=1,
+                             num_attention_heads=1, num_key_value_heads=1, head_dim=128, intermediate_size=16384,
+                             vocab_size=256, tied_lm_head=False, weight_seed=41)
+    p = W.ensure_model(wl, model_root())
+    if kind == "f32":
+        p = variant(p, model_root(), "f32")
+    g = T.Model.load(p)
+    n, cut = 262208, 262144
+    ids = T.synth_tokens(43, n, wl.vocab_size)
+    c = T.KvCache(g, n)
+    print("one call", flush=True)
+    whole = g.forward_seq(ids, c)
+    c.reset()
+    print("two calls", flush=True)
+    g.forward_seq(ids[:cut], c)
+    close_logits(g.forward_seq(ids[cut:], c), whole, "rows past 2^32 elements")
+    c.close()
+    g.close()

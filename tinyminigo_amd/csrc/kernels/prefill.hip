@@ -546,15 +546,17 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_span_kernel(const GemmArgs 
         }
         {
             const int row = wave * 16 + (lane >> 2);
-            boff = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
+            boff = (uint32_t)min(row, a.N - 1 - n0) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
         }
+        // 32-bit offsets within the tile's rows: all N of them may pass 2^32 elements
+        const uint16_t *const bhi = a.Bhi + (size_t)n0 * K, *const blo = a.Blo + (size_t)n0 * K;
         auto issue = [&](int st) {
             unsigned char *dst = smem + (st % kTStages) * kTStage;
 #pragma unroll
             for (int i = 0; i < WPW; i++)
                 __builtin_amdgcn_global_load_lds(a.W + woff[i] + st * kTK, dst + (wave * WPW + i) * 1024, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(a.Bhi + boff + st * kTK, dst + kTWTile + wave * 1024, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(a.Blo + boff + st * kTK, dst + kTWTile + kTBTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(bhi + boff + st * kTK, dst + kTWTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(blo + boff + st * kTK, dst + kTWTile + kTBTile + wave * 1024, 16, 0, 0);
         };
         // at most `n` later steps' DMAs may be outstanding (only DMAs are, and
         // they complete in issue order)
@@ -770,15 +772,17 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_f32w_span_kernel(const Gemm
         }
         {
             const int row = wave * 16 + (lane >> 2);
-            boff = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
+            boff = (uint32_t)min(row, a.N - 1 - n0) * (uint32_t)K + k0 * kTK + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
         }
+        // 32-bit offsets within the tile's rows: all N of them may pass 2^32 elements
+        const uint16_t *const bhi = a.Bhi + (size_t)n0 * K, *const blo = a.Blo + (size_t)n0 * K;
         auto issue = [&](int st) {
             unsigned char *dst = smem + (st % kFStages) * kFStage;
 #pragma unroll
             for (int i = 0; i < WPW; i++)
                 __builtin_amdgcn_global_load_lds(a.Wf + woff[i] + st * kTK, dst + (wave * WPW + i) * 1024, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(a.Bhi + boff + st * kTK, dst + kFWTile + wave * 1024, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(a.Blo + boff + st * kTK, dst + kFWTile + kTBTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(bhi + boff + st * kTK, dst + kFWTile + wave * 1024, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(blo + boff + st * kTK, dst + kFWTile + kTBTile + wave * 1024, 16, 0, 0);
         };
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -928,13 +932,15 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_dma_kernel(const GemmArgs a
         const int row = (wave * DPW + i) * 8 + (lane >> 3);
         const int lc = (lane & 7) ^ (row & 7);
         off[0][i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + lc * 8;
-        off[1][i] = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + lc * 8;
+        off[1][i] = (uint32_t)min(row, a.N - 1 - n0) * (uint32_t)K + lc * 8;
         off[2][i] = off[1][i];
     }
+    // 32-bit offsets within the tile's rows: all N of them may pass 2^32 elements
+    const uint16_t *const bhi = a.Bhi + (size_t)n0 * K, *const blo = a.Blo + (size_t)n0 * K;
     auto issue = [&](int stage, int k0) {
 #pragma unroll
         for (int x = 0; x < 3; x++) {
-            const uint16_t *base = x == 0 ? a.W : (x == 1 ? a.Bhi : a.Blo);
+            const uint16_t *base = x == 0 ? a.W : (x == 1 ? bhi : blo);
 #pragma unroll
             for (int i = 0; i < DPW; i++)
                 __builtin_amdgcn_global_load_lds(base + off[x][i] + k0,
@@ -1040,12 +1046,14 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_big_kernel(const GemmArgs a
         const int row = (wave * DPW + i) * 16 + (lane >> 2);
         const int lc = (lane & 3) ^ ((row >> 1) & 3);
         off[0][i] = (uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + lc * 8;
-        off[1][i] = (uint32_t)min(n0 + row, a.N - 1) * (uint32_t)K + lc * 8;
+        off[1][i] = (uint32_t)min(row, a.N - 1 - n0) * (uint32_t)K + lc * 8;
     }
+    // 32-bit offsets within the tile's rows: all N of them may pass 2^32 elements
+    const uint16_t *const bhi = a.Bhi + (size_t)n0 * K, *const blo = a.Blo + (size_t)n0 * K;
     auto issue = [&](int stage, int k0) {
 #pragma unroll
         for (int x = 0; x < 3; x++) {
-            const uint16_t *base = x == 0 ? a.W : (x == 1 ? a.Bhi : a.Blo);
+            const uint16_t *base = x == 0 ? a.W : (x == 1 ? bhi : blo);
 #pragma unroll
             for (int i = 0; i < DPW; i++)
                 __builtin_amdgcn_global_load_lds(base + off[x == 0 ? 0 : 1][i] + k0,
