@@ -258,6 +258,21 @@ typedef struct tmg_kernel_record {
 int tmg_profile_decode_step(tmg_model *model, tmg_cache *cache, uint32_t token, tmg_kernel_record *records,
                             size_t cap, size_t *n_records);
 
+/* The launch one kind of a prefill layer takes. */
+typedef struct tmg_plan_record {
+    char name[16];       /* "qkv", "attention", "o", "gate_up", "down" */
+    char kernel[32];     /* the kernel, e.g. "gemm_span", "attn_f32" */
+    uint32_t tiles;      /* its output tiles (attention: query tiles times KV heads) */
+    uint32_t workgroups; /* != tiles where a tile's K steps or keys are dealt to several */
+} tmg_plan_record;
+
+/* Which kernels a prefill of `tokens` tokens at position `start` takes, by the
+ * model's shapes alone (f32_weights: its matrices are F16 or F32): one record
+ * per kind of a layer's launch, in launch order.  Host only.  No counterpart in
+ * the reference (measurement only). */
+int tmg_prefill_plan(const tmg_config *cfg, int f32_weights, uint32_t tokens, uint32_t start,
+                     tmg_plan_record *records, size_t cap, size_t *n_records);
+
 typedef struct tmg_floor_record {
     char name[48];       /* kernel kind of the step */
     double bytes;        /* algorithmic HBM bytes of one launch of that kind */

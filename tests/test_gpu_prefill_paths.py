@@ -31,6 +31,8 @@ _open = {}
 
 
 def _models(mods, which):
+    if which in _SHAPES or which[4:] in _SHAPES:
+        return _shaped(mods, which)
     if which not in _open:
         T, O, W = mods
         if which.startswith("i8-"):
@@ -88,9 +90,9 @@ def _check(mods, which, pieces):
     gc2.close()
 
 
-# the tiled GEMM over spans of K steps: one token past a tile, a whole number
-# of tiles, past the short-prompt kernel's range, and lengths where spans cross
-# tiles and where tiles stay whole
+# lengths at and past the tiles' edges, whatever kernels they take (at 257 the
+# short-prompt ones alone, at 640 four different ones;
+# test_gemm_kernels_as_planned names the kernel of each of its cases)
 @pytest.mark.parametrize("which,n", [("1b", 257), ("1b", 577), ("1b", 640), ("1b", 1025), ("1b", 1408),
                                      ("h1088", 577), ("h1088", 1100)])
 def test_tiled_gemm_spans(mods, which, n):
@@ -256,3 +258,81 @@ def test_first_keys_at_minus_infinity(mods, pieces):
         at += m
     gc.close()
     g.close()
+
+
+_SHAPES = {
+    # two layers: the norm handed to QKV and from down
+    "1b-l2": dict(name="minicpm5-1b-synthetic-l2-v512", num_hidden_layers=2, vocab_size=512, weight_seed=31),
+    "4b-l2": dict(name="minicpm5-4b-synthetic-l2-v512", num_hidden_layers=2, vocab_size=512, weight_seed=47),
+    # row counts that end a quarter into a 256-row tile, and K that is an odd
+    # number of 32-wide steps there
+    "h1088-i4160": dict(name="llama-h1088-i4160-l1", num_hidden_layers=1, hidden_size=1088, num_attention_heads=8,
+                        num_key_value_heads=4, intermediate_size=4160, vocab_size=777, weight_seed=53),
+    "h1056": dict(name="llama-h1056-i2080-l1", num_hidden_layers=1, hidden_size=1056, num_attention_heads=8,
+                  num_key_value_heads=4, intermediate_size=2080, vocab_size=777, weight_seed=59),
+    # one and eight query heads per KV head
+    "g1": dict(name="llama-h512-q4-k4-l1", num_hidden_layers=1, hidden_size=512, num_attention_heads=4,
+               num_key_value_heads=4, intermediate_size=1024, vocab_size=777, weight_seed=61),
+    "g8": dict(name="llama-h512-q8-k1-l1", num_hidden_layers=1, hidden_size=512, num_attention_heads=8,
+               num_key_value_heads=1, intermediate_size=1024, vocab_size=777, weight_seed=67),
+}
+
+
+def _shaped(mods, which):
+    if which not in _open:
+        T, O, W = mods
+        f32 = which.startswith("f32-")
+        shape = which[4:] if f32 else which
+        wl = dataclasses.replace(W.FOUR_B if shape.startswith("4b") else W.ONE_B, **_SHAPES[shape])
+        p = W.ensure_model(wl, model_root())
+        if f32:
+            from f32models import variant
+            p = variant(p, model_root(), "f32")
+        _open[which] = T.Model.load(p), O.OracleModel.load(p), wl
+    return _open[which]
+
+
+def _plan(mods, which, n, start=0):
+    """{launch kind: (kernel, "whole" or "split")}; a line of tiles cut into
+    spans counts as split."""
+    T = mods[0]
+    plan = T.prefill_plan(_shaped(mods, which)[2], n, start, which.startswith("f32-"))
+    return {k: (kernel, "whole" if tiles == wgs else "split") for k, (kernel, tiles, wgs) in plan.items()}
+
+
+# every GEMM kernel above 64 tokens with each epilogue and norm hand-off that it
+# meets; the plan is asserted, so that a change of the estimates cannot leave a
+# case on another kernel
+@pytest.mark.parametrize("which,n,plan", [
+    ("1b-l2", 768, {"qkv": ("gemm_dma", "whole"), "o": ("gemm_skinny_wide", "whole"), "gate_up": ("gemm_span", "split"),
+                    "down": ("gemm_span", "split")}),
+    ("1b-l2", 1025, {"qkv": ("gemm_span", "whole"), "o": ("gemm_dma", "whole"), "gate_up": ("gemm_big", "whole"),
+                     "down": ("gemm_span", "split")}),
+    ("1b-l2", 2049, {"qkv": ("gemm_span", "split"), "o": ("gemm_span", "split"), "gate_up": ("gemm_big", "whole"),
+                     "down": ("gemm_span", "split")}),
+    ("1b-l2", 301, {"qkv": ("gemm_skinny_wide", "whole"), "o": ("gemm_skinny_pair", "whole"),
+                    "gate_up": ("gemm_skinny_wide", "whole"), "down": ("gemm_skinny_wide", "split")}),
+    ("4b-l2", 128, {"qkv": ("gemm_skinny_wide", "split"), "gate_up": ("gemm_span", "split")}),
+    ("4b-l2", 700, {"qkv": ("gemm_span", "split"), "o": ("gemm_skinny_wide", "whole"), "gate_up": ("gemm_big", "whole"),
+                    "down": ("gemm_span", "split")}),
+    ("h1088-i4160", 1025, {"qkv": ("gemm_dma", "whole"), "down": ("gemm_span", "split")}),
+    ("f32-h1056", 2, {k: ("gemm_f32w_span", "split") for k in ("qkv", "o", "gate_up", "down")}),
+    ("f32-h1056", 300, {k: ("gemm_f32w_span", "split") for k in ("qkv", "o", "gate_up", "down")}),
+])
+def test_gemm_kernels_as_planned(mods, which, n, plan):
+    got = _plan(mods, which, n)
+    assert {k: got[k] for k in plan} == plan
+    _check(mods, which, [n])
+
+
+# the attention kernels at every number of query heads per KV head, with the
+# keys of a query tile dealt to several workgroups: the fp32 kernel (a partial
+# column tile, one row), the split-bf16 one (a partial query block)
+@pytest.mark.parametrize("which", ["g1", "1b-l2", "4b-l2", "g8"])
+def test_attention_runs_per_group(mods, which):
+    pieces = [1000, 67, 300, 1]
+    at = pieces[0]
+    for n, kernel in zip(pieces[1:], ["attn_f32", "attn_prefill", "attn_f32"]):
+        assert _plan(mods, which, n, at)["attention"] == (kernel, "split")
+        at += n
+    _check(mods, which, pieces)

@@ -173,3 +173,16 @@ def test_tiny_model_file_fingerprint(tiny_path):
 def test_tokens_out_of_range_and_empty_prompt_checked_without_gpu():
     with pytest.raises(T.TmgError):
         T.Model.load("/nonexistent/model.safetensors")
+
+
+def test_prefill_plan():
+    plan = T.prefill_plan(W.ONE_B, 64)
+    assert list(plan) == ["qkv", "attention", "o", "gate_up", "down"]
+    # 192 whole 64 x 64 tiles; 64 query rows of 8 KV heads
+    assert plan["gate_up"] == ("gemm_skinny_pair", 192, 192) and plan["attention"] == ("attn_rows", 512, 512)
+    assert all(k.startswith("gemm_f32w") for n, (k, _, _) in T.prefill_plan(W.ONE_B, 64, f32_weights=True).items()
+               if n != "attention")
+    with pytest.raises(T.TmgError):
+        T.prefill_plan(W.ONE_B, 0)
+    with pytest.raises(T.TmgError):
+        T.prefill_plan(W.ONE_B, 1 << 30, 1)

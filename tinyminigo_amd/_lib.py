@@ -71,6 +71,10 @@ class tmg_kernel_record(C.Structure):
     _fields_ = [("name", C.c_char * 48), ("bytes", C.c_double), ("ms", C.c_float), ("launches", C.c_uint32)]
 
 
+class tmg_plan_record(C.Structure):
+    _fields_ = [("name", C.c_char * 16), ("kernel", C.c_char * 32), ("tiles", C.c_uint32), ("workgroups", C.c_uint32)]
+
+
 class tmg_floor_record(C.Structure):
     _fields_ = [("name", C.c_char * 48), ("bytes", C.c_double), ("floor_bytes", C.c_double), ("floor_ms", C.c_float),
                 ("launches", C.c_uint32), ("workgroups", C.c_uint32)]
@@ -132,6 +136,8 @@ SIGNATURES = {
     "tmg_gemv_i8": (C.c_int, [P, P, P, P, C.c_uint32, C.c_uint32, P]),
     "tmg_quantize_i8": (C.c_int, [P, C.c_uint32, C.c_uint32, P, P, P]),
     "tmg_decode_greedy": (C.c_int, [P, P, C.c_uint32, C.c_uint32, PU32, PF]),
+    "tmg_prefill_plan": (C.c_int, [C.POINTER(tmg_config), C.c_int, C.c_uint32, C.c_uint32, C.POINTER(tmg_plan_record),
+                                   C.c_size_t, C.POINTER(C.c_size_t)]),
     "tmg_profile_decode_step": (
         C.c_int, [P, P, C.c_uint32, C.POINTER(tmg_kernel_record), C.c_size_t, C.POINTER(C.c_size_t)]),
     "tmg_profile_step_floor": (

@@ -7,7 +7,9 @@
 #include <memory>
 #include <string>
 #include <cmath>
+#include <cstdio>
 #include <cstring>
+#include <utility>
 
 namespace tmg {
 
@@ -704,8 +706,9 @@ static int prefill_layers(tmg_model *m, int T, int start, float *k, float *v, ui
     // sums of squares, and QKV / gate-up apply the 1/rms scale in their
     // epilogues, instead of a separate normalization pass over the residual
     // (shapes permitting: hidden a multiple of 64, all four GEMMs on kernels
-    // with the staged epilogue)
-    // (f32 weight matrices run a per-element epilogue: no hand-off)
+    // with the staged epilogue).  Models with f32 weight matrices keep the
+    // separate pass: their GEMM's epilogue could carry the hand-off, which has
+    // not been measured there.
     bool f32_mats = false;
     for (const tmg_model::Layer &ly : m->layers) f32_mats = f32_mats || ly.qkv_f || ly.o_f || ly.gu_f || ly.down_f;
     const bool hand_off = !f32_mats && H % 256 == 0 && H / 64 <= kMaxNormGroups && gemm_stages_output(m->qkv_rows, T, H) &&
@@ -787,7 +790,7 @@ static int prefill_layers(tmg_model *m, int T, int start, float *k, float *v, ui
             aa.v_seq = rows->v;
             aa.kv_layer_off = layer_off;
             TMG_HIP(launch_attn(aa, s));
-        } else if (attn_prefill_supported(aa)) {
+        } else if (const PrefillKernel kind = plan_prefill_attn(aa).kernel; kind == kAttnMfma) {
             if ((rc = ensure_kv_split(m, start + T))) return rc;
             KVSplitArgs ka{kc, vc, start + T, m->nkv, m->hd, m->pf_kh, m->pf_kl, m->pf_vth, m->pf_vtl, m->kv_cap,
                            m->pf_vodd};
@@ -799,7 +802,7 @@ static int prefill_layers(tmg_model *m, int T, int start, float *k, float *v, ui
             aa.vt_pitch = m->kv_cap;
             aa.v_odd = m->pf_vodd;
             TMG_HIP(launch_attn_prefill(aa, s));
-        } else if (attn_f32_pays(aa)) {
+        } else if (kind == kAttnF32) {
             TMG_HIP(launch_attn_f32(aa, s));
         } else {
             TMG_HIP(launch_attn(aa, s));
@@ -1228,6 +1231,57 @@ extern "C" int tmg_decode_greedy(tmg_model *m, tmg_cache *c, uint32_t token, uin
     c->len += n_steps;
     if (ms) *ms = el;
     if (tokens_out && n_steps) memcpy(tokens_out, (const void *)c->history, (size_t)n_steps * 4);
+    return TMG_OK;
+}
+
+extern "C" int tmg_prefill_plan(const tmg_config *cfg, int f32_weights, uint32_t tokens, uint32_t start,
+                                tmg_plan_record *records, size_t cap, size_t *n_records) {
+    clear_error();
+    const uint64_t heads = cfg ? cfg->num_attention_heads : 0, kv = cfg ? cfg->num_key_value_heads : 0;
+    if (!cfg || !records || !n_records || !heads || !kv || heads % kv || !cfg->head_dim || !cfg->hidden_size ||
+        !cfg->intermediate_size || !tokens || heads > 16384 || cfg->head_dim > 16384 || cfg->hidden_size > 16384 ||
+        cfg->intermediate_size > 16384 || (uint64_t)tokens + start > 0x3fffffff)
+        return set_error(TMG_E_INVALID, "bad argument to tmg_prefill_plan");
+    static const char *const kernels[] = {"gemm", "gemm_skinny", "gemm_skinny_pair", "gemm_skinny_wide", "gemm_span",
+                                          "gemm_dma", "gemm_big", "gemm_f32w_span", "attn_rows", "attn_f32",
+                                          "attn_prefill"};
+    const int qd = (int)(heads * cfg->head_dim), kvd = (int)(kv * cfg->head_dim);
+    const int H = (int)cfg->hidden_size, I = (int)cfg->intermediate_size;
+    float scratch;  // stands for the workspaces, which a prefill always has
+    unsigned count;
+    uint16_t half;
+    auto gemm = [&](int M, int K) {
+        GemmArgs g{};
+        if (f32_weights) g.Wf = &scratch;
+        g.M = M;
+        g.N = (int)tokens;
+        g.K = K;
+        g.part = &scratch;
+        g.cnt = &count;
+        return plan_gemm(g);
+    };
+    AttnArgs aa{};
+    aa.nq = (int)heads;
+    aa.nkv = (int)kv;
+    aa.hd = (int)cfg->head_dim;
+    aa.T = (int)tokens;
+    aa.start = (int)start;
+    aa.out_hi = aa.out_lo = &half;
+    aa.part = aa.part_ml = &scratch;
+    const std::pair<const char *, LaunchPlan> plans[] = {{"qkv", gemm(qd + 2 * kvd, H)},
+                                                         {"attention", plan_prefill_attn(aa)},
+                                                         {"o", gemm(H, qd)},
+                                                         {"gate_up", gemm(2 * I, H)},
+                                                         {"down", gemm(H, I)}};
+    *n_records = 0;
+    for (const auto &p : plans) {
+        if (*n_records == cap) break;
+        tmg_plan_record &r = records[(*n_records)++];
+        snprintf(r.name, sizeof(r.name), "%s", p.first);
+        snprintf(r.kernel, sizeof(r.kernel), "%s", kernels[p.second.kernel]);
+        r.tiles = (uint32_t)p.second.tiles;
+        r.workgroups = (uint32_t)p.second.workgroups;
+    }
     return TMG_OK;
 }
 

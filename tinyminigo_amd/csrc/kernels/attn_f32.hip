@@ -301,6 +301,11 @@ bool attn_f32_pays(const AttnArgs &a) {
     return 11.0 + std::max(2.6 * run, 2.0 * run * wgs / 256.0) + (nsp > 1 ? 6.0 : 0.0) < rows_us;
 }
 
+LaunchPlan attn_f32_plan(const AttnArgs &a) {
+    const int cols = kFCols / (a.nq / a.nkv), tiles = (a.T + cols - 1) / cols * a.nkv;
+    return LaunchPlan{kAttnF32, tiles, tiles * f32_runs(a)};
+}
+
 hipError_t launch_attn_f32(const AttnArgs &a, hipStream_t s) {
     if (a.T <= 0 || a.hd != kFHD || !a.out_hi || !a.out_lo || a.pos_seq) return hipErrorInvalidValue;
     switch (a.nq / a.nkv) {

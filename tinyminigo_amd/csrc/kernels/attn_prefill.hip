@@ -644,6 +644,15 @@ bool attn_prefill_supported(const AttnArgs &a) {
     return a.T >= kTiledMinTokens;
 }
 
+LaunchPlan plan_prefill_attn(const AttnArgs &a) {
+    if (attn_prefill_supported(a)) {
+        const int QB = kPCols / (a.nq / a.nkv);
+        return LaunchPlan{kAttnMfma, (a.T + QB - 1) / QB * a.nkv, plan_attn(a).workgroups};
+    }
+    if (attn_f32_pays(a)) return attn_f32_plan(a);
+    return LaunchPlan{kAttnRows, a.T * a.nkv, a.T * a.nkv};
+}
+
 hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s) {
     if (!attn_prefill_supported(a) || a.T <= 0 || !a.kh || !a.kl || !a.vth || !a.vtl ||
         !a.v_odd || !a.k_cache || !a.v_cache || a.vt_pitch < (a.start + a.T + kPKB - 1) / kPKB * kPKB || a.vt_pitch % 8)

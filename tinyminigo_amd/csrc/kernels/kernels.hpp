@@ -103,6 +103,28 @@ hipError_t launch_quantize_i8_f32(const float *w, int rows, int in, int8_t *q8, 
 // (BF16 rows, or f32 rows with f32).
 int gemv_blocks(int out, int in, bool f32 = false);
 
+// The kernel that a prefill launch takes, its output tiles (attention: query
+// tiles times KV heads) and its workgroups: more than tiles where a tile's K
+// steps or keys are dealt to several, fewer or more where the tiles' K steps
+// are cut into spans (equal to the tiles where every span is a whole tile).
+enum PrefillKernel {
+    kGemmStream,      // gemm_kernel
+    kGemmSkinny,      // gemm_skinny_kernel
+    kGemmSkinnyPair,  // gemm_skinny_kernel, step pairs
+    kGemmSkinnyWide,  // gemm_skinny_wide_kernel
+    kGemmSpan,        // gemm_span_kernel
+    kGemmDma,         // gemm_dma_kernel
+    kGemmBig,         // gemm_big_kernel
+    kGemmF32Span,     // gemm_f32w_span_kernel
+    kAttnRows,        // attn_kernel
+    kAttnF32,         // attn_f32_kernel
+    kAttnMfma,        // attn_prefill_kernel
+};
+struct LaunchPlan {
+    PrefillKernel kernel;
+    int tiles, workgroups;
+};
+
 struct AttnArgs {
     const float *q;  // [T][nq*hd], RoPE applied
     const float *k_cache, *v_cache;  // layer base, [pos][nkv*hd]
@@ -163,7 +185,10 @@ hipError_t launch_attn_prefill(const AttnArgs &a, hipStream_t s);
 // column tile's keys may be dealt to several workgroups.
 constexpr int kAttnF32Runs = 512;
 bool attn_f32_pays(const AttnArgs &a);
+LaunchPlan attn_f32_plan(const AttnArgs &a);
 hipError_t launch_attn_f32(const AttnArgs &a, hipStream_t s);
+// Which of the three one sequence's prefill attention takes.
+LaunchPlan plan_prefill_attn(const AttnArgs &a);
 // Merges the split-K partials of a decode attention launch (a.T rows) into
 // out_f32 [T][nq*hd]: where the merge is not fused into the o_proj GEMV
 // prologue (more than kFusedSplits splits; batched decode).
@@ -260,12 +285,14 @@ struct GemmArgs {
     unsigned *cnt;
 };
 
-// Prompts of at least kTiledMinTokens tokens may take the 256 x 256 GEMM tile,
-// and their attention the MFMA kernel; up to kShortMaxTokens tokens the
-// split-K kernel of short prompts (launch_gemm chooses by estimated time).
+// Prompts of at least kTiledMinTokens tokens may take the 256 x 256 and the
+// 128 x 128 GEMM tile, and their attention the MFMA kernel; up to
+// kShortMaxTokens tokens the split-K kernels of short prompts (plan_gemm chooses
+// by estimated time).
 constexpr int kTiledMinTokens = 256;
 constexpr int kShortMaxTokens = 1024;
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s);
+LaunchPlan plan_gemm(const GemmArgs &a);
 // Whether launch_gemm takes a kernel whose output goes through
 // stage_epilogue for these shapes (the only ones that honour nrm_w / nss_in).
 bool gemm_stages_output(int M, int N, int K);

@@ -1459,7 +1459,8 @@ __global__ __launch_bounds__(2 * kBlock, 1) void gemm_skinny_wide_kernel(const G
                                        out, &pre);
 }
 
-// K splits of gemm_skinny_wide_kernel
+// K splits of gemm_skinny_wide_kernel: while the grid stays within one
+// workgroup (eight waves, a 96 KB ring) per CU, at least 2 steps per split
 int skinny_wide_splits(const GemmArgs &a) {
     const int m2 = (a.M + 127) / 128, n_tiles = (a.N + 63) / 64, nk = a.K / 64;
     int ns = 1;
@@ -1468,10 +1469,10 @@ int skinny_wide_splits(const GemmArgs &a) {
     return ns;
 }
 
-hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
-    // split K while the grid stays within one workgroup per CU, or while
-    // splits keep at least 20 K steps within three workgroups per CU; at most
-    // kSkMaxSplit ways, at least 2 steps per split
+// K splits of gemm_skinny_kernel: while the grid stays within one workgroup
+// per CU, or while splits keep at least 20 K steps within three workgroups per
+// CU; at most kSkMaxSplit ways, at least 2 steps per split
+int skinny_splits(const GemmArgs &a) {
     const int m_tiles = (a.M + 63) / 64, n_tiles = (a.N + 63) / 64, nk = a.K / 64;
     int nsplit = 1;
     if (a.part && a.cnt) {
@@ -1484,11 +1485,28 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
                 break;
         }
     }
+    return nsplit;
+}
+
+// The split-K kernels of short prompts.  Step pairs (PAIR) where K is not split
+// and the 64-row grid is at most one workgroup per CU, at any token count;
+// else 64-row tiles of four waves for one token tile (128-row tiles measured
+// slower there: 1B 64-token prefill 1.62 -> 1.81 ms), and 128-row tiles for
+// two or more (the activation tiles staged once per 128 weight rows; 4B
+// 128-token prefill 5.83 -> 5.58 ms).
+LaunchPlan plan_skinny(const GemmArgs &a) {
+    const int n_tiles = (a.N + 63) / 64, tiles = (a.M + 63) / 64 * n_tiles, nsplit = skinny_splits(a);
+    if (nsplit == 1 && tiles <= 256) return LaunchPlan{kGemmSkinnyPair, tiles, tiles};
+    if (n_tiles == 1) return LaunchPlan{kGemmSkinny, tiles, tiles * nsplit};
+    const int tiles2 = (a.M + 127) / 128 * n_tiles;
+    return LaunchPlan{kGemmSkinnyWide, tiles2, tiles2 * skinny_wide_splits(a)};
+}
+
+hipError_t launch_skinny(int epi, const GemmArgs &a, const LaunchPlan &p, hipStream_t s) {
+    const int m_tiles = (a.M + 63) / 64, n_tiles = (a.N + 63) / 64, nsplit = p.workgroups / p.tiles;
     if (nsplit > 1 && (size_t)m_tiles * n_tiles * nsplit * 4096 > kSkinnyPartFloats) return hipErrorInvalidValue;
     const dim3 grid((m_tiles * nsplit + 7) / 8 * n_tiles * 8);
-    // eight wavefronts per workgroup (step pairs) where K is not split and the
-    // grid is at most one workgroup per CU
-    if (nsplit == 1 && m_tiles * n_tiles <= 256) {
+    if (p.kernel == kGemmSkinnyPair) {
         switch (epi) {
             case GEPI_STORE: hipLaunchKernelGGL((gemm_skinny_kernel<GEPI_STORE, true>), grid, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
             case GEPI_RESID: hipLaunchKernelGGL((gemm_skinny_kernel<GEPI_RESID, true>), grid, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
@@ -1498,9 +1516,7 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
         }
         return hipGetLastError();
     }
-    // one token tile: 64-row tiles of four waves (128-row tiles measured
-    // slower there: 1B 64-token prefill 1.62 -> 1.81 ms)
-    if (n_tiles == 1) {
+    if (p.kernel == kGemmSkinny) {
         switch (epi) {
             case GEPI_STORE: hipLaunchKernelGGL((gemm_skinny_kernel<GEPI_STORE, false>), grid, dim3(kBlock), 0, s, a, nsplit, n_tiles); break;
             case GEPI_RESID: hipLaunchKernelGGL((gemm_skinny_kernel<GEPI_RESID, false>), grid, dim3(kBlock), 0, s, a, nsplit, n_tiles); break;
@@ -1510,19 +1526,13 @@ hipError_t launch_skinny(int epi, const GemmArgs &a, hipStream_t s) {
         }
         return hipGetLastError();
     }
-    // two or more token tiles: 128-row tiles (the activation tiles staged
-    // once per 128 weight rows; 4B 128-token prefill 5.83 -> 5.58 ms), K
-    // split while the grid stays within one workgroup (eight waves, a 96 KB
-    // ring) per CU
     const int m2 = (a.M + 127) / 128;
-    const int ns2 = skinny_wide_splits(a);
-    if (ns2 > 1 && (size_t)m_tiles * n_tiles * ns2 * 4096 > kSkinnyPartFloats) return hipErrorInvalidValue;
-    const dim3 grid2((m2 * ns2 + 7) / 8 * n_tiles * 8);
+    const dim3 grid2((m2 * nsplit + 7) / 8 * n_tiles * 8);
     switch (epi) {
-        case GEPI_STORE: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_STORE>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
-        case GEPI_RESID: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_RESID>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
-        case GEPI_SWIGLU: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_SWIGLU>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
-        case GEPI_QKV: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_QKV>), grid2, dim3(2 * kBlock), 0, s, a, ns2, n_tiles); break;
+        case GEPI_STORE: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_STORE>), grid2, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
+        case GEPI_RESID: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_RESID>), grid2, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
+        case GEPI_SWIGLU: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_SWIGLU>), grid2, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
+        case GEPI_QKV: hipLaunchKernelGGL((gemm_skinny_wide_kernel<GEPI_QKV>), grid2, dim3(2 * kBlock), 0, s, a, nsplit, n_tiles); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1587,11 +1597,10 @@ SpanPlan plan_span(const GemmArgs &a) {
     return p;
 }
 
-hipError_t launch_span(int epi, const GemmArgs &a, hipStream_t s) {
-    const int m_tiles = (a.M + kTM - 1) / kTM, n_tiles = (a.N + kTN - 1) / kTN, nk = a.K / kTK;
-    const int tiles = m_tiles * n_tiles;
+hipError_t launch_span(int epi, const GemmArgs &a, const LaunchPlan &p, hipStream_t s) {
+    const int n_tiles = (a.N + kTN - 1) / kTN, nk = a.K / kTK, tiles = p.tiles, G = p.workgroups;
     if ((int64_t)tiles * nk > 0x3fffffff) return hipErrorInvalidValue;
-    const int units = tiles * nk, G = plan_span(a).spans;
+    const int units = tiles * nk;
     const SpanCut cut{n_tiles, nk, units / G, units % G};
     switch (epi) {
         case GEPI_STORE: launch_span_epi<GEPI_STORE>(a, cut, tiles, G, s); break;
@@ -1633,43 +1642,66 @@ bool gemm_stages_output(int M, int N, int K) {
     return K % 64 == 0 || (K % 32 == 0 && N >= kTiledMinTokens && big_fills(M, N));
 }
 
+LaunchPlan plan_gemm(const GemmArgs &a) {
+    const int span_tiles = ((a.M + kTM - 1) / kTM) * ((a.N + kTN - 1) / kTN);
+    if (a.Wf) return LaunchPlan{kGemmF32Span, span_tiles, plan_span(a).spans};
+    const bool tiled = a.K % 64 == 0 && a.N > 64;
+    const SpanPlan span = tiled ? plan_span(a) : SpanPlan{0, HUGE_VAL};
+    const double short_us = tiled && a.N <= kShortMaxTokens ? skinny_wide_us(a) : HUGE_VAL;
+    if (a.N >= kTiledMinTokens && (tiled ? big_us(a) < std::min({span.us, short_us, dma_us(a)}) : big_fills(a.M, a.N))) {
+        const int wg = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
+        return LaunchPlan{kGemmBig, wg, wg};
+    }
+    if (tiled && a.N >= kTiledMinTokens && dma_us(a) < std::min(span.us, short_us)) {
+        const int wg = ((a.M + kDM - 1) / kDM) * ((a.N + kDN - 1) / kDN);
+        return LaunchPlan{kGemmDma, wg, wg};
+    }
+    if (tiled && span.us < short_us) return LaunchPlan{kGemmSpan, span_tiles, span.spans};
+    if (a.K % 64 == 0) return plan_skinny(a);
+    const int wg = ((a.M + 15) / 16) * ((a.N + 63) / 64);
+    return LaunchPlan{kGemmStream, wg, wg};
+}
+
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     if (a.K % 32 != 0 || a.M <= 0 || a.N <= 0) return hipErrorInvalidValue;
-    if (a.Wf) {
-        // f32 weights: the per-element epilogue only (no norm hand-off, no row scales)
-        if (a.nrm_w || a.nss_in || a.wscale) return hipErrorInvalidValue;
-        return launch_span(epi, a, s);
-    }
+    // the launches over f32 weights take no row scales, and no norm hand-off:
+    // their epilogue could, but the callers normalize in a pass of its own
+    // there (the hand-off has not been measured with it)
+    if (a.Wf && (a.nrm_w || a.nss_in || a.wscale)) return hipErrorInvalidValue;
     if ((a.nrm_w || a.nss_in) && !gemm_stages_output(a.M, a.N, a.K)) return hipErrorInvalidValue;
     if (a.nrm_w && (epi != GEPI_RESID || a.M % 64 != 0 || !a.nss || !a.nx_hi || !a.nx_lo)) return hipErrorInvalidValue;
     if (a.nss_in && (a.ngroups <= 0 || a.ngroups > kMaxNormGroups || a.ngroups % 4)) return hipErrorInvalidValue;
-    const bool tiled = a.K % 64 == 0 && a.N > 64;
-    const double span_us = tiled ? plan_span(a).us : HUGE_VAL;
-    const double short_us = tiled && a.N <= kShortMaxTokens ? skinny_wide_us(a) : HUGE_VAL;
-    if (a.N >= kTiledMinTokens && (tiled ? big_us(a) < std::min({span_us, short_us, dma_us(a)}) : big_fills(a.M, a.N))) {
-        const dim3 grid((a.M + kBM - 1) / kBM, (a.N + kBN - 1) / kBN);
-        switch (epi) {
-            case GEPI_STORE: hipLaunchKernelGGL(gemm_big_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_RESID: hipLaunchKernelGGL(gemm_big_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_big_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_QKV: hipLaunchKernelGGL(gemm_big_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            default: return hipErrorInvalidValue;
+    const LaunchPlan p = plan_gemm(a);
+    switch (p.kernel) {
+        case kGemmF32Span:
+        case kGemmSpan: return launch_span(epi, a, p, s);
+        case kGemmBig: {
+            const dim3 grid((a.M + kBM - 1) / kBM, (a.N + kBN - 1) / kBN);
+            switch (epi) {
+                case GEPI_STORE: hipLaunchKernelGGL(gemm_big_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_RESID: hipLaunchKernelGGL(gemm_big_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_big_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_QKV: hipLaunchKernelGGL(gemm_big_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                default: return hipErrorInvalidValue;
+            }
+            return hipGetLastError();
         }
-        return hipGetLastError();
-    }
-    if (tiled && a.N >= kTiledMinTokens && dma_us(a) < std::min(span_us, short_us)) {
-        const dim3 grid((a.M + kDM - 1) / kDM, (a.N + kDN - 1) / kDN);
-        switch (epi) {
-            case GEPI_STORE: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_RESID: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            case GEPI_QKV: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
-            default: return hipErrorInvalidValue;
+        case kGemmDma: {
+            const dim3 grid((a.M + kDM - 1) / kDM, (a.N + kDN - 1) / kDN);
+            switch (epi) {
+                case GEPI_STORE: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_STORE>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_RESID: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_RESID>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_SWIGLU: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_SWIGLU>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                case GEPI_QKV: hipLaunchKernelGGL(gemm_dma_kernel<GEPI_QKV>, grid, dim3(kGWaves * 64), 0, s, a); break;
+                default: return hipErrorInvalidValue;
+            }
+            return hipGetLastError();
         }
-        return hipGetLastError();
+        case kGemmSkinny:
+        case kGemmSkinnyPair:
+        case kGemmSkinnyWide: return launch_skinny(epi, a, p, s);
+        default: break;
     }
-    if (tiled && span_us < short_us) return launch_span(epi, a, s);
-    if (a.K % 64 == 0) return launch_skinny(epi, a, s);
     const dim3 grid((a.M + 15) / 16, (a.N + 63) / 64);
     switch (epi) {
         case GEPI_STORE: hipLaunchKernelGGL(gemm_kernel<GEPI_STORE>, grid, dim3(kBlock), 0, s, a); break;

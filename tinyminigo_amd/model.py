@@ -18,12 +18,12 @@ import weakref
 
 from ._lib import (
     ON_TOKEN, TmgError, check, finalizing, lib, register, tmg_config, tmg_floor_record, tmg_gen_params,
-    tmg_kernel_record, tmg_synth_spec,
+    tmg_kernel_record, tmg_plan_record, tmg_synth_spec,
 )
 
 __all__ = [
     "ModelConfig", "Model", "KvCache", "GenParams", "GenOutput", "generate", "gemv_bf16", "gemv_i8", "quantize_i8", "repack_tmb",
-    "argmax_f32", "profile_stream",
+    "argmax_f32", "prefill_plan", "profile_stream",
     "generate_batch",
     "synth_model", "synth_tokens", "synth_normal_bf16", "synth_normal_f32", "TmgError",
 ]
@@ -274,6 +274,17 @@ def generate(model: Model, prompt_tokens: Sequence[int], params: GenParams,
         raise err[0]
     return GenOutput(tokens=[int(x) for x in out[:n_out.value]], logits_first_step=first,
                      prefill_secs=secs.value)
+
+
+def prefill_plan(config, tokens: int, start: int = 0, f32_weights: bool = False) -> dict:
+    """tmg_prefill_plan: {launch kind: (kernel, tiles, workgroups)} of a prefill
+    layer; config is anything with the model's sizes as attributes."""
+    cfg = tmg_config()
+    for name in ("hidden_size", "num_attention_heads", "num_key_value_heads", "head_dim", "intermediate_size"):
+        setattr(cfg, name, getattr(config, name))
+    recs, n = (tmg_plan_record * 8)(), C.c_size_t()
+    check(lib.tmg_prefill_plan(C.byref(cfg), int(f32_weights), int(tokens), int(start), recs, len(recs), C.byref(n)))
+    return {r.name.decode(): (r.kernel.decode(), r.tiles, r.workgroups) for r in recs[:n.value]}
 
 
 def profile_stream(nbytes: int, wg_kib: int, device: int = 0):
