@@ -186,3 +186,12 @@ def test_prefill_plan():
         T.prefill_plan(W.ONE_B, 0)
     with pytest.raises(T.TmgError):
         T.prefill_plan(W.ONE_B, 1 << 30, 1)
+
+
+def test_attention_of_short_prompts_counts_each_rows_own_context():
+    # 160 rows from position 0 read 288 chunks of 64 positions per KV head, not
+    # 160 x 3, and the per-row kernel is the faster one; after a long context it
+    # is not
+    assert T.prefill_plan(W.ONE_B, 160)["attention"][0] == "attn_rows"
+    assert T.prefill_plan(W.ONE_B, 255)["attention"][0] == "attn_f32"
+    assert T.prefill_plan(W.ONE_B, 160, 1000)["attention"][0] == "attn_f32"

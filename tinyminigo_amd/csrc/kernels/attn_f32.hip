@@ -291,11 +291,19 @@ bool attn_f32_pays(const AttnArgs &a) {
         !(group == 1 || group == 2 || group == 4 || group == 8))
         return false;
     // The per-row kernel: 1.66 us per 64 positions of one round of workgroups,
-    // 200 such chunks per us once the chip is full.  This one: 2.6 us per
-    // block of a run, 2 us per block and 256 workgroups once it is full, 11 us
-    // for the launch, first loads and merge, 6 us for merging runs.
+    // 200 such chunks per us (300 with one query head per KV head) once the chip
+    // is full, each row those up to its own position (with the last row's count
+    // for all, this kernel was taken where it was slower: the 1B shape at 145-180
+    // tokens by 2% of the prefill, one query head per KV head by 8-10%).  With
+    // four or more query heads its chunks are 16 positions and slower, and the
+    // last row's count stands for that.  This one: 2.6 us per block of a run, 2 us
+    // per block and 256 workgroups once it is full, 11 us for the launch, first
+    // loads and merge, 6 us for merging runs.
     const double chunks = (a.start + a.T + 63) / 64;
-    const double rows_us = 3.0 + std::max(1.66 * chunks, (double)a.T * a.nkv * chunks / 200.0);
+    // chunks of rows 0 .. n - 1
+    auto below = [](int64_t n) { return 32 * (n / 64) * (n / 64 - 1) + n / 64 * (n % 64) + n; };
+    const double all = group < 4 ? (double)(below(a.start + a.T) - below(a.start)) : a.T * chunks;
+    const double rows_us = 3.0 + std::max(1.66 * chunks, all * a.nkv / (group == 1 ? 300.0 : 200.0));
     const int nsp = f32_runs(a), tiles = (a.T + kFCols / group - 1) / (kFCols / group);
     const double run = std::max(1.0, chunks / nsp), wgs = (double)tiles * nsp * a.nkv;
     return 11.0 + std::max(2.6 * run, 2.0 * run * wgs / 256.0) + (nsp > 1 ? 6.0 : 0.0) < rows_us;
