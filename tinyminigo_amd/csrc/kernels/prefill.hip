@@ -1155,8 +1155,9 @@ __global__ __launch_bounds__(kGWaves * 64) void gemm_big_kernel(const GemmArgs a
                                 n0 + wn * 64, acc);
 }
 
-// Split-K MFMA GEMM for short prompts (up to 64 tokens; the 128-row form below up
-// to kShortMaxTokens).
+// Split-K MFMA GEMM for short prompts: up to 64 tokens, and in its PAIR form any
+// unsplit grid of at most 256 tiles (plan_skinny); the 128-row form below takes
+// the other prompts up to kShortMaxTokens.
 //
 // Workgroup tile: 64 weight rows x 64 tokens over one contiguous range of K
 // (split ks of nsplit).  Each 64-wide K step's W, Bhi and Blo tiles go
@@ -1547,19 +1548,27 @@ void launch_span_epi(const GemmArgs &a, const SpanCut &cut, int tiles, int G, hi
     if (G != tiles) hipLaunchKernelGGL(gemm_span_reduce_kernel<EPI>, dim3(tiles * 8), dim3(kBlock), 0, s, a, cut);
 }
 
-// Estimated microseconds of a GEMM on the four kernels that take more than 64
-// tokens, from kernel traces of the 1B and 4B shapes at 75-8192 tokens.  Each
-// is a fixed cost (launch, ring fill, epilogue) plus the K steps of the
-// longest workgroup: a 64-wide step of the 128 x 128 tile takes 1.02 us, 1.2
-// where several rounds keep the chip full; a 32-wide step of the 256 x 128
-// tile 1.1 us (0.95 in one round of whole tiles), of the 256 x 256 tile 1.8; a 64-wide step of the 128 x 64 tile
-// 0.6-0.75.  A K split of the short-prompt kernel costs about 5 us for its
-// exchange, one of the span kernel about 8 us plus 0.06 us per span (128 KB of
-// partials written and read back).  Choosing by them instead of by token count
-// (256 x 256 from 240 tiles, 128 x 128 from 256 tokens) and with the span
-// kernel, the 1B prefill went from 6.6 to 3.95 ms at 301 tokens, 7.0 to 4.5 at
-// 500, 11.9 to 10.9 at 1500, the 4B prefill from 14.5 to 7.7 at 300 and 18.0
-// to 15.9 at 700.
+// Estimated microseconds of a GEMM of more than 64 tokens on each kernel, from
+// kernel traces of the 1B and 4B shapes at 75-8192 tokens.  Each is a fixed cost
+// (launch, ring fill, epilogue) plus the K steps of the longest workgroup: a
+// 64-wide step of the 128 x 128 tile takes 1.02 us, 1.2 where several rounds
+// keep the chip full; a 32-wide step of the 256 x 128 tile 1.1 us (0.95 in one
+// round of whole tiles), of the 256 x 256 tile 1.8; a 64-wide step of the
+// 128 x 64 tile 0.6-0.75.  A K split of the short-prompt kernel costs about 5 us
+// for its exchange, one of the span kernel about 8 us plus 0.06 us per span
+// (128 KB of partials written and read back).
+//
+// The short-prompt line is that of the 128-row kernel.  It is high where
+// plan_skinny takes the PAIR form instead (1B o_proj at 301 tokens: 22 us
+// estimated, 16.9 measured; QKV at 130: 22 and 18.4) and for long K splits (1B
+// down at 301: 45 and 36), so near a crossover the span and 128 x 128 kernels
+// are taken a little too early.
+//
+// Choosing by these lines instead of by token count (256 x 256 from 240 tiles,
+// 128 x 128 from 256 tokens): 1B 6.6 -> 3.95 ms at 301 tokens, all of it from the
+// short-prompt kernels, 7.0 -> 4.5 at 500 (the gate/up on whole 256 x 128 tiles)
+// and 11.9 -> 10.9 at 1500 (split spans for the gate/up); 4B 14.5 -> 7.7 at 300
+// and 18.0 -> 15.9 at 700 (split spans for QKV and down).
 double big_us(const GemmArgs &a) {
     const int wg = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
     return 8.0 + 1.8 * ((wg + 255) / 256) * (a.K / kBK);
