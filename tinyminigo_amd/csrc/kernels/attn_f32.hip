@@ -33,27 +33,10 @@ namespace tmg {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kFHD = 128;   // head dim
 constexpr int kFCols = 32;  // query columns per workgroup, two MFMA column tiles
 constexpr int kFKB = 64;    // keys per block, 16 per wavefront
-
-__device__ __forceinline__ float max_groups(float v) {  // over the four lane groups of a column
-    auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
-    s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
-}
-
-// 16 consecutive output dims (o[e][i] is dim 4 i + e), scaled, as split-bf16
-__device__ __forceinline__ void store_dims4(const f32x4 &v, uint16_t *hi, uint16_t *lo) {
-    uint16_t h[4], l[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) split_bf16(v[e], h + e, l + e);
-    *reinterpret_cast<u32x2 *>(hi) = u32x2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    *reinterpret_cast<u32x2 *>(lo) = u32x2{(uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16)};
-}
 
 // Workgroup (tile * nsp + sp) * nkv + g: run sp of column tile `tile`.
 template <int GROUP>
@@ -122,7 +105,7 @@ __global__ __launch_bounds__(kBlock, 2) void attn_f32_kernel(const AttnArgs a, i
                 for (int i = 0; i < 4; i++)
                     if (k0 + 4 * q4 + i > qpos[ct]) s[ct][i] = -INFINITY;
             }
-            const float mx = max_groups(fmaxf(fmaxf(s[ct][0], s[ct][1]), fmaxf(s[ct][2], s[ct][3])));
+            const float mx = max_xor16_32(fmaxf(fmaxf(s[ct][0], s[ct][1]), fmaxf(s[ct][2], s[ct][3])));
             // the maximum is raised in steps of at least 2^8 (see attn_prefill_kernel)
             const bool raise = mx > m[ct] + 8.0f;
             if (__builtin_amdgcn_ballot_w64(raise)) {
@@ -225,7 +208,7 @@ __global__ __launch_bounds__(kBlock, 2) void attn_f32_kernel(const AttnArgs a, i
     const float inv = 1.0f / L;
     const size_t ob = (size_t)ti * qd + (g * GROUP + c % GROUP) * kFHD + 64 * h + 16 * q4;
 #pragma unroll
-    for (int i = 0; i < 4; i++) store_dims4(out[i] * inv, a.out_hi + ob + 4 * i, a.out_lo + ob + 4 * i);
+    for (int i = 0; i < 4; i++) store_split4(out[i] * inv, a.out_hi + ob + 4 * i, a.out_lo + ob + 4 * i);
 }
 
 // Merges the runs of a column tile in key order: workgroup (tile * 4 + i) *
@@ -265,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void attn_f32_combine_kernel(const AttnArgs
     }
     if (ti >= a.T) return;
     const size_t ob = (size_t)ti * (a.nq * kFHD) + (g * GROUP + c % GROUP) * kFHD + 64 * h + 16 * q4 + 4 * i;
-    store_dims4(o * (1.0f / L), a.out_hi + ob, a.out_lo + ob);
+    store_split4(o * (1.0f / L), a.out_hi + ob, a.out_lo + ob);
 }
 
 // Runs per column tile: two workgroups per CU, a run at least one block.

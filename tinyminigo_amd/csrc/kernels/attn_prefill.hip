@@ -77,18 +77,6 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 &hi, bf16x8 &
     lo = __builtin_bit_cast(bf16x8, l);
 }
 
-__device__ __forceinline__ float max_xor16_32(float v) {
-    {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-    {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-    return v;
-}
-
 // Slot of a key (its position within its 64-key block) in a V^T row.  The
 // P^T operand of O^T += V^T P^T gives lane (q4, r) the keys 4 q4 .. +3 of two
 // adjacent 16-key tiles; within each 32-key group those eight keys are
@@ -181,15 +169,6 @@ __host__ __device__ inline int key_blocks(int start, int T, int QB, int qb) {
     return last / kPKB + 1;
 }
 __host__ __device__ inline int key_splits(int nkb, int run) { return (nkb + run - 1) / run; }
-
-// Four consecutive output dims as split-bf16.
-__device__ __forceinline__ void store_split4(const f32x4 &v, uint16_t *hi, uint16_t *lo) {
-    uint16_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) split_bf16(v[i], h + i, l + i);
-    *reinterpret_cast<u32x2 *>(hi) = u32x2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    *reinterpret_cast<u32x2 *>(lo) = u32x2{(uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16)};
-}
 
 template <int GROUP>
 __global__ __launch_bounds__(kPWaves * 64) void attn_prefill_kernel(const AttnArgs a) {

@@ -27,6 +27,16 @@ __device__ __forceinline__ void split_bf16(float x, uint16_t *hi, uint16_t *lo) 
     *lo = f32_to_bf16_rne(x - bf16_to_f32(h));
 }
 
+// Four consecutive values as split-bf16, 8 bytes to each plane.
+template <class F4>
+__device__ __forceinline__ void store_split4(const F4 &v, uint16_t *hi, uint16_t *lo) {
+    uint16_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) split_bf16(v[i], h + i, l + i);
+    *reinterpret_cast<uint2 *>(hi) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    *reinterpret_cast<uint2 *>(lo) = make_uint2((uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16));
+}
+
 // Cross-lane moves without LDS: DPP within rows of 16 lanes and the gfx950
 // permlane swaps across rows.  For lane l:
 //   xor1 / xor2      -> value of lane l^1 / l^2       (DPP quad_perm)
@@ -82,20 +92,20 @@ __device__ __forceinline__ T group_sum(T v) {
 
 __device__ __forceinline__ float wave_sum(float v) { return group_sum<64>(v); }
 
+// The maximum over lanes l, l^16, l^32 and l^48.
+__device__ __forceinline__ float max_xor16_32(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, dpp_mov<kDppXor1>(v));
     v = fmaxf(v, dpp_mov<kDppXor2>(v));
     v = fmaxf(v, dpp_mov<kDppHalfMirror>(v));
     v = fmaxf(v, dpp_mov<kDppRor8>(v));
-    {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-    {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    }
-    return v;
+    return max_xor16_32(v);
 }
 
 // log2 of a power-of-two count of values per lane, at most 64 (one per lane).
