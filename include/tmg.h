@@ -83,8 +83,9 @@ int tmg_config_load(const char *config_json_path, tmg_config *out);
  * (src/config.rs:174-184).  BF16 weight matrices are uploaded raw to HBM on
  * `device`; F16 and F32 ones are widened to f32 rows (WMat::F32,
  * src/model.rs:49-55) and multiplied as f32 (tmg_gemv_f32's arithmetic in
- * decode, an fp32 GEMM in prefill).  Norm weights and the embedding may be
- * BF16, F16 or F32 (converted as in src/safetensors_loader.rs:103-147).  With
+ * decode, exact products of the f32 weights in the prefill GEMM).  Norm
+ * weights and the embedding may be BF16, F16 or F32 (converted as in
+ * src/safetensors_loader.rs:103-147).  With
  * TMG_I8=1 in the environment (the reference's gate, src/model.rs:57-76) the
  * q, k, v, o, gate, up and down projections are quantized to per-row int8 at
  * load (tmg_quantize_i8, from the f32 values for F16/F32 matrices): decode

@@ -1,7 +1,7 @@
 """F32 / F16 weight matrices on the GPU (WMat::F32: the reference converts
 such tensors to f32 at load, src/model.rs:49-55, and multiplies them with
-`dot`, src/tensor.rs:58-74 and 387-420): the f32-row decode GEMV, the fp32
-MFMA prefill GEMM and the loader, against the oracle's f32 path on the same
+`dot`, src/tensor.rs:58-74 and 387-420): the f32-row decode GEMV, the
+prefill GEMM over split f32 weights and the loader, against the oracle's f32 path on the same
 files.  Tolerances are the decode path's (logits within 2e-3 abs + 1e-3 rel,
 greedy ids identical)."""
 import dataclasses
@@ -132,8 +132,8 @@ def test_tied_f32_embedding_vs_oracle(T, O, tiny_path):
 
 def test_f32_long_prompt_and_wide_heads(T, O, W):
     # hidden 2048, head_dim 128 (the 1B shapes, 2 layers, vocab 1024): a
-    # 300-token prompt takes the fp32-MFMA GEMM at K = 2048 and 6144 and the
-    # MFMA prefill attention; decode the f32-row GEMVs at one and three chunks
+    # 300-token prompt takes the GEMM over f32 weights at K = 2048 and 6144 and
+    # the MFMA prefill attention; decode the f32-row GEMVs at one and three chunks
     wl = dataclasses.replace(W.ONE_B, name="mid-h2048-l2-v1024", num_hidden_layers=2, vocab_size=1024,
                              weight_seed=17)
     p = variant(W.ensure_model(wl, model_root()), model_root(), "f32")

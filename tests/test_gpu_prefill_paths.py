@@ -1,8 +1,9 @@
 """Prefill kernels at the edges of their tiles and splits, against the oracle.
 
-One-layer models: the 1B model's layer, whose GEMMs leave tiles in parts at
-these lengths, and one whose row counts are odd multiples of 64 (the last
-256-row tile is mostly past the edge).
+One-layer models: the 1B and 4B models' layers and one whose row counts are odd
+multiples of 64 (the last 256-row tile is mostly past the edge).  Two-layer
+ones where the norm handed between GEMMs counts, and small ones for the other
+head groupings.
 """
 import dataclasses
 import os
